@@ -39,10 +39,10 @@ int ensure_buffer(kp_ctx* c, void** buf, size_t* cap, size_t bytes) {
     return KP_OK;
 }
 
-// Largest persistent grid of any traversal launch: the spill area has one
-// slice per lane of it.
+// Largest grid of any traversal launch (the integrator's pair launches hold
+// both 5-wave grids): the spill area has one slice per lane of it.
 uint32_t max_trace_grid(const kp_ctx* c) {
-    return std::max(std::max(c->grid_closest, c->grid_occluded), std::max(c->grid_closest5, c->grid_occluded5));
+    return std::max(std::max(c->grid_closest, c->grid_occluded), c->grid_closest5 + c->grid_occluded5);
 }
 
 TraceArgs trace_base(kp_ctx* c) {
@@ -77,7 +77,7 @@ int trace_closest_dev(kp_ctx* c, const float4* rays, uint32_t n, float4* hits, b
     // variant has a 4-wave kernel of its own
     const bool five = !count;
     a.five_waves = five ? 1u : 0u;
-    hipError_t e = launch_closest(a, five ? c->grid_closest5 : c->grid_closest, count, c->stream);
+    hipError_t e = launch_closest(a, five ? c->grid_closest5 : c->grid_closest, count, true, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "closest-hit launch");
     return KP_OK;
 }
@@ -916,7 +916,7 @@ int kp_intersect_closest_noalloc(kp_ctx* c, const kp_ray* rays, uint32_t n, kp_h
     a.spill_blocks = grid;
     c->noalloc_used = true;
     KP_HIP_TRY(c, kp::launch_reset_u32(a.err, 1u, c->stream));   // launch_closest clears the counter
-    hipError_t e = kp::launch_closest(a, grid, false, c->stream);
+    hipError_t e = kp::launch_closest(a, grid, false, true, c->stream);
     if (e != hipSuccess) return kp::hip_fail(c, e, "kp_intersect_closest_noalloc launch");
     return KP_OK;
 }

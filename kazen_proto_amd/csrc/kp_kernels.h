@@ -45,9 +45,28 @@ struct TraceArgs {
     // one-level closest / occluded launches of the integrator: the kernels
     // compiled for 5 waves per SIMD (96 registers) instead of 4
     uint32_t five_waves;
+    // connecting occlusion (set inside the pair kernel): per ray its
+    // contribution and path slot, per slot the radiance it is added to
+    const float4* scontrib;
+    float4* radiance;
 };
 
-hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, hipStream_t s);
+// The shadow queue of a pair launch (the rest as in its TraceArgs).
+struct ShadowQueue {
+    const float4* rays;
+    const uint32_t* n_dev;
+    uint32_t* counter;
+    const uint32_t* roots;
+    const float4* contrib;   // {rgb, path slot bits} per ray
+    float4* radiance;        // per path slot
+};
+
+// reset: clear the work counter first (otherwise the caller has cleared it)
+hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool reset, hipStream_t s);
+// Closest hit of a (grid_closest blocks) and the connecting occlusion of q
+// (grid_occluded blocks) in one launch; both work counters already cleared.
+hipError_t launch_pair(const TraceArgs& a, const ShadowQueue& q, uint32_t grid_closest, uint32_t grid_occluded,
+                       hipStream_t s);
 hipError_t launch_occluded(const TraceArgs& a, uint32_t grid, hipStream_t s);
 hipError_t trace_occupancy(int* blocks_per_cu_closest, int* blocks_per_cu_occluded);
 hipError_t trace_occupancy_five(int* blocks_per_cu_closest, int* blocks_per_cu_occluded);

@@ -7,14 +7,21 @@
 //
 // One pass traces k samples of every pixel as n = width*height*k independent
 // paths (slot = pixel*k + j).  Per bounce:
-//   extend  : closest hit of the compacted ray queue (trace.hip)
+//   trace   : closest hit of the compacted ray queue and, from the second
+//             bounce on, in the same launch the occlusion of the shadow rays
+//             of the vertices before; contributions of unoccluded ones are
+//             added to their paths by the traversal (trace.hip)
 //   shade   : emission with MIS, next-event estimation (writes a shadow ray),
 //             Russian roulette, BSDF sampling (writes the next ray); both
 //             queues are compacted with a ballot per wave and one atomic per
 //             block and queue (same-address device atomics are the limit:
 //             one per wave made shading 3.4x slower)
-//   connect : occlusion of the shadow queue, then the unoccluded
-//             contributions are added to their paths
+// Two launches a bounce.  A launch costs 4 to 5 us even when it has next to
+// nothing to do, and a traversal launch ends with a drain of 30 to 50 us, so
+// with closest hit, occlusion, connect, and counter clearing each launched on
+// their own (eight a bounce) a 160 x 120 preview at depth 5 took 746 us and
+// now takes 458; 256 x 256 at 16 samples 1,706 and 1,354; 1024 x 1024 at 16
+// samples of a two-million-triangle terrain at depth 8 16.59 and 15.25 ms.
 // After the last bounce every pixel folds its k path radiances into the film
 // (FP32 sum with Kahan compensation, one owner per pixel, fixed order), so
 // the film does not depend on scheduling.
@@ -60,18 +67,25 @@ struct PathState {
     uint64_t* rng;        // per slot: PCG32 state
     float4* srays;        // shadow queue rays
     float4* scontrib;     // shadow contribution.xyz, slot bits in w
-    uint32_t* socc;       // occlusion result per shadow ray
-    uint32_t* cnt;        // queue sizes qc(0), qc(1) rays, qc(2) shadow rays
+    uint32_t* cnt;        // queue sizes and traversal work counters of every bounce, cleared by generate
     unsigned long long* totals;   // [0] extension rays, [1] shadow rays
     // batched scenes only
     uint32_t* slot_scene; // per slot: scene of the path
     uint32_t* slot_pixel; // per slot: pixel of the path in its scene
     uint32_t* qroot[2];   // per ray-queue entry: BVH root of the ray's scene
     uint32_t* sroot;      // per shadow-queue entry: BVH root
-    // Each queue counter has a 256-byte line of its own: the two counters
-    // one shade appends to are then served by different memory channels.
-    __host__ __device__ uint32_t& qc(uint32_t i) const { return cnt[i * 64u]; }
+    // Each counter has a 256-byte line of its own: the two counters one shade
+    // appends to are then served by different memory channels.  Every bounce
+    // has its own four, so one clearing per pass serves all its launches.
+    __host__ __device__ uint32_t* line(uint32_t depth, uint32_t k) const { return cnt + (4u * depth + k) * 64u; }
+    __host__ __device__ uint32_t* rays_at(uint32_t depth) const { return line(depth, 0); }      // ray queue size
+    __host__ __device__ uint32_t* shadows_at(uint32_t depth) const { return line(depth, 1); }   // shadow queue size
+    __host__ __device__ uint32_t* ray_work(uint32_t depth) const { return line(depth, 2); }     // traversal counters
+    __host__ __device__ uint32_t* shadow_work(uint32_t depth) const { return line(depth, 3); }
 };
+// Depths 1 .. KP_MAX_DEPTH + 1 have counters (and 0 and one more as padding).
+#define KP_MAX_DEPTH 64u
+#define KP_COUNTER_LINES (4u * (KP_MAX_DEPTH + 3u))
 
 // One scene of a batch (the camera, film and sampling settings of its
 // kp_render_desc, its BVH root and light range in the merged arrays).  Work
@@ -97,6 +111,7 @@ struct RenderArgs {
     uint32_t width, height, npix, k, n_paths;
     uint32_t seq_base;       // PCG sequence of slot s = seq_base + s / k
     uint32_t seed, s0, max_depth, rr_depth;
+    uint32_t first_pass;     // the call's first pass clears the ray totals
     float3 eye, fwd, right, upv;
     float tan_half, aspect;
     PathState ps;
@@ -170,14 +185,28 @@ __device__ __forceinline__ uint32_t cdf_sample(const float* cdf, uint32_t count,
 }
 
 // ------------------------------------------------------------- kernels --
+// First kernel of a pass: its first block clears every bounce's counters, sets
+// the first queue's size and, in a call's first pass, clears the ray totals.
+__device__ __forceinline__ void start_pass(const PathState& ps, uint32_t n, bool first) {
+    if (blockIdx.x != 0) return;
+    for (uint32_t i = threadIdx.x; i < KP_COUNTER_LINES; i += 256)
+        ps.cnt[i * 64u] = ps.cnt + i * 64u == ps.rays_at(1) ? n : 0u;
+    if (first && threadIdx.x < 2) ps.totals[threadIdx.x] = 0ull;
+}
+
+// Last kernel of a pass: its first block adds the queue sizes to the totals.
+__device__ __forceinline__ void end_pass(const PathState& ps, uint32_t max_depth) {
+    if (blockIdx.x != 0) return;
+    for (uint32_t d = 1 + threadIdx.x; d <= max_depth + 1; d += 256) {
+        atomicAdd(&ps.totals[0], (unsigned long long)*ps.rays_at(d));
+        atomicAdd(&ps.totals[1], (unsigned long long)*ps.shadows_at(d));
+    }
+}
+
 __global__ __launch_bounds__(256) void k_generate(RenderArgs a) {
 #pragma clang fp contract(off)
     const uint32_t slot = blockIdx.x * 256 + threadIdx.x;
-    if (slot == 0) {
-        a.ps.qc(0) = a.n_paths;
-        a.ps.qc(1) = 0;
-        a.ps.qc(2) = 0;
-    }
+    start_pass(a.ps, a.n_paths, a.first_pass);
     if (slot >= a.n_paths) return;
     const uint32_t pixel = slot / a.k;
     const uint32_t j = slot - pixel * a.k;
@@ -204,11 +233,7 @@ __global__ __launch_bounds__(256) void k_generate(RenderArgs a) {
 // rays): sequence = seq_base + slot, sample index = s0.
 __global__ __launch_bounds__(256) void k_generate_rays(RenderArgs a, const float4* rays) {
     const uint32_t slot = blockIdx.x * 256 + threadIdx.x;
-    if (slot == 0) {
-        a.ps.qc(0) = a.n_paths;
-        a.ps.qc(1) = 0;
-        a.ps.qc(2) = 0;
-    }
+    start_pass(a.ps, a.n_paths, a.first_pass);
     if (slot >= a.n_paths) return;
     const uint64_t initstate = ((uint64_t)a.s0 << 32) ^ (uint64_t)a.seed ^ 0x9E3779B97F4A7C15ull;
     const Pcg rng = pcg_seed(initstate, a.seq_base + slot);
@@ -234,11 +259,7 @@ __global__ __launch_bounds__(256) void k_generate_batch(RenderArgs a) {
 #pragma clang fp contract(off)
     const uint32_t slot = blockIdx.x * 256 + threadIdx.x;
     const uint32_t n = batch_pass_paths(a);
-    if (slot == 0) {
-        a.ps.qc(0) = n;
-        a.ps.qc(1) = 0;
-        a.ps.qc(2) = 0;
-    }
+    start_pass(a.ps, n, a.pass[0] == 0);
     if (slot >= n) return;
     const unsigned long long w = a.pass[0] + slot;
     uint32_t lo = 0, hi = a.n_scenes;   // last scene with work_first <= w
@@ -287,6 +308,7 @@ __global__ __launch_bounds__(256) void k_film_batch(RenderArgs a, float4* sum, f
     const uint32_t base = blockIdx.x * 256;
     const uint32_t t = threadIdx.x, slot = base + t;
     const uint32_t n = batch_pass_paths(a);
+    end_pass(a.ps, a.max_depth);
     if (slot < n) {
         xs[t] = a.ps.s1[slot];
         ss[t + 1] = a.ps.slot_scene[slot];
@@ -366,24 +388,12 @@ __global__ void k_rebase_lights(LightRec* l, uint32_t n, uint32_t lt_off, uint32
 
 __global__ void k_write_radiance(RenderArgs a, float* out) {
     const uint32_t slot = blockIdx.x * 256 + threadIdx.x;
+    end_pass(a.ps, a.max_depth);
     if (slot >= a.n_paths) return;
     const float4 l = a.ps.s1[slot];
     out[3 * (size_t)slot] = l.x;
     out[3 * (size_t)slot + 1] = l.y;
     out[3 * (size_t)slot + 2] = l.z;
-}
-
-// Resets the output queue counters of the coming shade, accumulating totals.
-__global__ void k_bookkeep(RenderArgs a, int cur) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        a.ps.totals[0] += a.ps.qc(cur);
-        a.ps.qc(cur ^ 1) = 0;
-        a.ps.qc(2) = 0;
-    }
-}
-
-__global__ void k_count_shadow(RenderArgs a) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) a.ps.totals[1] += a.ps.qc(2);
 }
 
 // Appends the lanes with `want0` to queue c0 and those with `want1` to queue
@@ -428,7 +438,7 @@ __global__ __launch_bounds__(256) void k_shade(RenderArgs a, int cur, uint32_t d
     __shared__ uint32_t n_blk;
     // one read of the queue size per block: the loop below synchronises the
     // block every iteration, so all its threads must agree on the trip count
-    if (threadIdx.x == 0) n_blk = a.ps.qc(cur);
+    if (threadIdx.x == 0) n_blk = *a.ps.rays_at(depth);
     __syncthreads();
     const uint32_t n = n_blk;
     const uint32_t total = gridDim.x * 256;
@@ -694,7 +704,7 @@ __global__ __launch_bounds__(256) void k_shade(RenderArgs a, int cur, uint32_t d
             a.ps.rng[slot] = rng.state;
         }
         uint32_t so;
-        const uint32_t qo = block_append2(cont, shad, &a.ps.qc(cur ^ 1), &a.ps.qc(2), app_lds, so);
+        const uint32_t qo = block_append2(cont, shad, a.ps.rays_at(depth + 1), a.ps.shadows_at(depth), app_lds, so);
         if (cont) {
             rout[2 * (size_t)qo] = nr0;
             rout[2 * (size_t)qo + 1] = nr1;
@@ -707,21 +717,6 @@ __global__ __launch_bounds__(256) void k_shade(RenderArgs a, int cur, uint32_t d
             a.ps.scontrib[so] = sc;
             if (a.scenes) a.ps.sroot[so] = root;
         }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_connect(RenderArgs a) {
-    const uint32_t n = a.ps.qc(2);
-    const uint32_t total = gridDim.x * 256;
-    for (uint32_t s = blockIdx.x * 256 + threadIdx.x; s < n; s += total) {
-        if (a.ps.socc[s]) continue;
-        const float4 c = a.ps.scontrib[s];
-        const uint32_t slot = __float_as_uint(c.w);
-        float4 l = a.ps.s1[slot];
-        l.x += c.x;
-        l.y += c.y;
-        l.z += c.z;
-        a.ps.s1[slot] = l;
     }
 }
 
@@ -772,6 +767,7 @@ __global__ __launch_bounds__(256) void k_guide_records(RenderArgs a, uint32_t n_
 __global__ __launch_bounds__(256) void k_film(RenderArgs a, float4* sum, float4* comp) {
 #pragma clang fp contract(off)
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+    end_pass(a.ps, a.max_depth);
     if (p >= a.npix) return;
     float4 s = sum[p], c = comp[p];
     for (uint32_t j = 0; j < a.k; ++j) {
@@ -1044,14 +1040,14 @@ static int alloc_paths(kp_ctx* c, PathState& ps, void*& mem, uint32_t& cap, uint
     mem = nullptr;
     cap = 0;
     // bytes per slot: 2x32 rays + 2x4 qmap + 16 hit + 16 s0 + 16 s1 + 8 rng
-    //                 + 32 shadow ray + 16 contrib + 4 occl
+    //                 + 32 shadow ray + 16 contrib
     //                 + 5x4 batch (scene, pixel, roots of the three queues)
     const size_t N = n;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~size_t(255); return o; };
     const size_t o_r0 = take(N * 32), o_r1 = take(N * 32), o_q0 = take(N * 4), o_q1 = take(N * 4);
     const size_t o_h = take(N * 16), o_s0 = take(N * 16), o_s1 = take(N * 16), o_rng = take(N * 8);
-    const size_t o_sr = take(N * 32), o_sc = take(N * 16), o_so = take(N * 4), o_cnt = take(3 * 256),
+    const size_t o_sr = take(N * 32), o_sc = take(N * 16), o_cnt = take(KP_COUNTER_LINES * 256),
                  o_tot = take(64);
     const size_t o_ss = take(N * 4), o_sp = take(N * 4), o_qr0 = take(N * 4), o_qr1 = take(N * 4),
                  o_sr2 = take(N * 4);
@@ -1067,7 +1063,6 @@ static int alloc_paths(kp_ctx* c, PathState& ps, void*& mem, uint32_t& cap, uint
     ps.rng = (uint64_t*)(b + o_rng);
     ps.srays = (float4*)(b + o_sr);
     ps.scontrib = (float4*)(b + o_sc);
-    ps.socc = (uint32_t*)(b + o_so);
     ps.cnt = (uint32_t*)(b + o_cnt);
     ps.totals = (unsigned long long*)(b + o_tot);
     ps.slot_scene = (uint32_t*)(b + o_ss);
@@ -1075,11 +1070,6 @@ static int alloc_paths(kp_ctx* c, PathState& ps, void*& mem, uint32_t& cap, uint
     ps.qroot[0] = (uint32_t*)(b + o_qr0);
     ps.qroot[1] = (uint32_t*)(b + o_qr1);
     ps.sroot = (uint32_t*)(b + o_sr2);
-    // on the context's stream (created non-blocking: null-stream work would
-    // not be ordered with its kernels), never inside a captured graph
-    KP_HIP_TRY(c, hipMemsetAsync(ps.cnt, 0, 3 * 256, c->stream));
-    KP_HIP_TRY(c, hipMemsetAsync(ps.totals, 0, 64, c->stream));
-    KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
     cap = n;
     return KP_OK;
 }
@@ -1166,9 +1156,12 @@ static TraceCfg ctx_trace_cfg(kp_ctx* c) {
     return t;
 }
 
-// Extend / shade / connect for max_depth + 1 bounces of the paths that the
-// generate kernel has queued (queue sizes live on the device).  Only kernel
-// launches: the sequence can be captured into a graph.
+// Trace / shade for max_depth + 1 bounces of the paths that the generate
+// kernel has queued (queue sizes live on the device).  From the second bounce
+// on a trace launch holds the path rays and the shadow rays of the vertices
+// before them; the shadow rays' contributions are in the radiance when the
+// bounce is shaded.  Only kernel launches: the sequence can be captured into
+// a graph.
 static int run_bounces(kp_ctx* c, const RenderArgs& a, bool guided, const TraceCfg& tc, uint32_t max_depth) {
     int cur = 0;
     for (uint32_t depth = 1; depth <= max_depth + 1; ++depth) {
@@ -1176,26 +1169,26 @@ static int run_bounces(kp_ctx* c, const RenderArgs& a, bool guided, const TraceC
         ta.rays = a.ps.rays[cur];
         ta.hits = a.ps.hits;
         ta.n = a.n_paths;
-        ta.n_dev = &a.ps.qc(cur);
+        ta.n_dev = a.ps.rays_at(depth);
+        ta.counter = a.ps.ray_work(depth);
         ta.roots = tc.roots ? a.ps.qroot[cur] : nullptr;
-        KP_HIP_TRY(c, launch_closest(ta, tc.grid_closest, false, c->stream));
-        hipLaunchKernelGGL(k_bookkeep, dim3(1), dim3(64), 0, c->stream, a, cur);
+        if (depth == 1) {
+            KP_HIP_TRY(c, launch_closest(ta, tc.grid_closest, false, false, c->stream));
+        } else {
+            ShadowQueue q;
+            q.rays = a.ps.srays;
+            q.n_dev = a.ps.shadows_at(depth - 1);
+            q.counter = a.ps.shadow_work(depth - 1);
+            q.roots = tc.roots ? a.ps.sroot : nullptr;
+            q.contrib = a.ps.scontrib;
+            q.radiance = a.ps.s1;
+            KP_HIP_TRY(c, launch_pair(ta, q, tc.grid_closest, tc.grid_occluded, c->stream));
+        }
         if (guided)
             hipLaunchKernelGGL(k_shade<true>, dim3(tc.shade_blocks_guided), dim3(256), 0, c->stream, a, cur, depth);
         else
             hipLaunchKernelGGL(k_shade<false>, dim3(tc.shade_blocks), dim3(256), 0, c->stream, a, cur, depth);
         KP_HIP_TRY(c, hipGetLastError());
-        if (depth <= max_depth) {
-            ta.rays = a.ps.srays;
-            ta.hits = nullptr;
-            ta.occl = a.ps.socc;
-            ta.n_dev = &a.ps.qc(2);
-            ta.roots = tc.roots ? a.ps.sroot : nullptr;
-            KP_HIP_TRY(c, launch_occluded(ta, tc.grid_occluded, c->stream));
-            hipLaunchKernelGGL(k_count_shadow, dim3(1), dim3(64), 0, c->stream, a);
-            hipLaunchKernelGGL(k_connect, dim3(tc.shade_blocks), dim3(256), 0, c->stream, a);
-            KP_HIP_TRY(c, hipGetLastError());
-        }
         cur ^= 1;
     }
     return KP_OK;
@@ -1258,14 +1251,13 @@ static int integrate_rays(kp_ctx* c, const kp_ray* rays, uint32_t n, const kp_re
         d_in = (float4*)c->d_stage_in;
         d_out = (float*)c->d_stage_out;
     }
-    unsigned long long zero2[2] = {0, 0};
-    KP_HIP_TRY(c, hipMemcpyAsync(r->ps.totals, zero2, 16, hipMemcpyHostToDevice, c->stream));
     auto t0 = std::chrono::steady_clock::now();
     for (uint32_t off = 0; off < n; off += cap) {
         const uint32_t cnt = (n - off) < cap ? (n - off) : cap;
         RenderArgs a = base_render_args(c);
         a.k = 1;
         a.n_paths = cnt;
+        a.first_pass = off == 0 ? 1u : 0u;
         a.seq_base = off;
         a.s0 = d->spp_offset;
         a.seed = d->seed;
@@ -1359,10 +1351,9 @@ static int render_accumulate(kp_ctx* c, const kp_render_desc* d) {
     bool train = false;
     uint32_t pass_steps = 0;
     auto t0 = std::chrono::steady_clock::now();
-    unsigned long long zero2[2] = {0, 0};
-    KP_HIP_TRY(c, hipMemcpyAsync(r->ps.totals, zero2, 16, hipMemcpyHostToDevice, c->stream));
     for (uint32_t pass = 0; pass < d->spp / k; ++pass) {
         a.s0 = d->spp_offset + pass * k;
+        a.first_pass = pass == 0 ? 1u : 0u;
         uint32_t n_rec = 0;
         if (guided) {
             a.guide_on = g->train_passes >= g->guide_after ? 1u : 0u;
@@ -1727,8 +1718,6 @@ static int batch_render(BatchState* b, const kp_render_desc* descs, uint32_t max
     int rc = alloc_paths(c, b->ps, b->path_mem, b->cap_paths, chunk);
     if (rc) return rc;
     if (b->path_mem != old_mem || b->cap_paths != old_cap) batch_drop_graph(b);
-    unsigned long long zero2[2] = {0, 0};
-    KP_HIP_TRY(c, hipMemcpy(b->ps.totals, zero2, 16, hipMemcpyHostToDevice));
     RenderArgs a{};
     a.stris = b->stris;
     a.snorm = b->snorm;

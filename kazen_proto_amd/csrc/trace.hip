@@ -353,6 +353,7 @@ constexpr uint32_t kTailChunk = 64;
 struct RayFeeder {
     uint32_t next, end, n;
     uint32_t dyn_base;  // first ray handed out by the counter (after the static chunks)
+    uint32_t waves;     // waves that share the queue
     bool drained;
     uint32_t* counter;
     const float4* rays;
@@ -360,7 +361,9 @@ struct RayFeeder {
     uint32_t pid, proot;   // prefetched ray of this lane (pid KP_INVALID: none) and its root
     float4 p0, p1;
 
-    __device__ __forceinline__ void init(uint32_t* ctr, const float4* rs, const uint32_t* rts, uint32_t count) {
+    // block / blocks: this block's index among the blocks that share the queue
+    __device__ __forceinline__ void init(uint32_t* ctr, const float4* rs, const uint32_t* rts, uint32_t count,
+                                         uint32_t block, uint32_t blocks) {
         counter = ctr;
         rays = rs;
         roots = rts;
@@ -371,8 +374,8 @@ struct RayFeeder {
         // (every wave of the grid would otherwise hit the one counter address
         // at start); the counter hands out the rays after all first chunks,
         // and a wave whose first chunk lies beyond the rays has none.
-        const uint32_t waves = gridDim.x * (blockDim.x >> 6);
-        const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+        waves = blocks * (KP_TRACE_BLOCK / 64);
+        const uint32_t wave = block * (KP_TRACE_BLOCK / 64) + (threadIdx.x >> 6);
         // up to kChunk rays per wave: every ray in a first chunk (multiples of
         // 64, as many waves as that takes); more: the first chunks hold
         // about half the rays (256 .. 4096 per wave) and the counter's chunks
@@ -407,7 +410,7 @@ struct RayFeeder {
             }
             // the last chunk taken ended at `end`: small chunks once fewer
             // than kChunk rays per wave were left after it
-            const uint64_t late = (uint64_t)(gridDim.x * (blockDim.x >> 6)) * kChunk;
+            const uint64_t late = (uint64_t)waves * kChunk;
             const uint32_t size = (uint64_t)end + late >= n ? kTailChunk : kChunk;
             uint32_t base = 0;
             if (__lane_id() == 0) base = atomicAdd(counter, size);
@@ -444,7 +447,13 @@ constexpr uint32_t kStuckBatch = 8u;
 struct LeafLds {
     uint32_t map[KP_TRACE_BLOCK];             // wave's 64 entries: owner lane << 8 | item of the owner
     unsigned long long key[KP_TRACE_BLOCK];   // closest hit: minimum hit key; any hit: nonzero once hit
-    float4 hit[KP_TRACE_BLOCK];               // closest hit: {t, u, v} of the minimum key
+    union {
+        float4 hit[KP_TRACE_BLOCK];           // closest hit: {t, u, v} of the minimum key
+        struct {                              // any hit, connecting: rays found unoccluded
+            uint32_t n[KP_TRACE_BLOCK / 64];
+            uint32_t ray[KP_TRACE_BLOCK / 64][128];   // < 64 left over + at most one per lane and pass
+        } open;
+    };
 };
 
 __device__ __forceinline__ unsigned long long hit_key(float t, uint32_t prim);
@@ -604,12 +613,57 @@ __device__ __forceinline__ uint32_t nth_set_bit(unsigned long long m, uint32_t r
     return pos + (r >= ((uint32_t)m & 1u) ? 1u : 0u);
 }
 
+// LDS of one traversal block (31 KB, so five blocks fit a CU).  Split rays
+// (one level) and world-space rays (two-level) never meet in one kernel.
+struct SplitLds {
+    unsigned long long key[KP_TRACE_BLOCK];       // owner: minimum helper hit key
+    float4 hit[KP_TRACE_BLOCK];                   // owner: {t, u, v} of that key
+    uint32_t role[KP_TRACE_BLOCK];                // owner thread | kHelper | kDonated | kWaiting
+    unsigned long long busy[KP_TRACE_BLOCK / 64];   // wave: owners with helpers at work
+};
+struct TraceLds {
+    uint2 stack[KP_TRACE_STACK][KP_TRACE_BLOCK];
+    LeafLds leaf;
+    union {
+        SplitLds split;
+        float4 wray[2][KP_TRACE_BLOCK];   // world ray per lane (two-level)
+    };
+};
+
 // Lane roles of a split closest-hit ray (low 8 bits: block thread of the
 // lane that owns the ray).
 constexpr uint32_t kHelper = 1u << 8;    // traverses a group of another lane's ray
 constexpr uint32_t kDonated = 1u << 9;   // owner whose ray has had groups handed out
 constexpr uint32_t kWaiting = 1u << 10;  // owner done with its part, helpers still at work
 constexpr uint32_t kStepsWaiting = 0xFFFFFFFFu;   // step count of a waiting owner (skips the traversal)
+
+// Rays on the wave's list of unoccluded ones (written by any of its lanes).
+__device__ __forceinline__ uint32_t open_count(LeafLds& L, int tid) {
+    return __hip_atomic_load(&L.open.n[tid >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+__device__ __forceinline__ void set_open_count(LeafLds& L, int tid, uint32_t n) {
+    __hip_atomic_store(&L.open.n[tid >> 6], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// Adds the contributions of up to 64 of the wave's listed unoccluded rays to
+// their paths (the last ones of the list) and shortens the list.  Every lane
+// of the wave must call it.
+__device__ __forceinline__ void connect_open(const TraceArgs& args, LeafLds& L, uint32_t open, int tid) {
+    const uint32_t left = open > 64u ? open - 64u : 0u;
+    const uint32_t i = left + __lane_id();
+    if (i < open) {
+        const float4 c = args.scontrib[L.open.ray[tid >> 6][i]];
+        float4* l = args.radiance + __float_as_uint(c.w);
+        float4 x = *l;
+        x.x += c.x;
+        x.y += c.y;
+        x.z += c.z;
+        *l = x;
+    }
+    __builtin_amdgcn_wave_barrier();
+    set_open_count(L, tid, left);
+    __builtin_amdgcn_wave_barrier();
+}
 
 // Persistent traversal shared by closest hit (kAny = false) and occlusion
 // (kAny = true).  A node visit tests the 8 children; the nearest hit inner
@@ -648,20 +702,25 @@ constexpr uint32_t kStepsWaiting = 0xFFFFFFFFu;   // step count of a waiting own
 // without splitting.  A helper also culls with its owner's closest distance
 // once that is nearer (read at every pass of the drain phase).  Occlusion
 // does not split: split occlusion rays made the integrator 2 % slower.
-template <bool kAny, bool kCount, bool kInst>
-__device__ __forceinline__ void traverse(const TraceArgs& args) {
-    __shared__ uint2 lds[kStack][KP_TRACE_BLOCK];
-    __shared__ LeafLds leafl;
-    __shared__ float4 wray[kInst ? 2 : 1][kInst ? KP_TRACE_BLOCK : 1];   // world ray per lane (two-level)
+//
+// Connect (kConnect, occlusion): instead of a flag per ray, a ray that is not
+// occluded adds its contribution to its path's radiance.  The finished rays
+// are listed in LDS and added 64 at a time, so the two dependent loads
+// (contribution, radiance) are waited for once per 64 rays, not once per
+// loop pass.  A path has at most one ray in the queue: no two adds meet.
+template <bool kAny, bool kCount, bool kInst, bool kConnect = false>
+__device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uint32_t block, uint32_t blocks) {
     constexpr bool kSplit = !kAny && !kInst;
-    __shared__ unsigned long long skey[kSplit ? KP_TRACE_BLOCK : 1];      // owner: minimum helper hit key
-    __shared__ float4 shit[kSplit ? KP_TRACE_BLOCK : 1];                  // owner: {t, u, v} of that key
-    __shared__ uint32_t srole[kSplit ? KP_TRACE_BLOCK : 1];               // owner thread | kHelper | kDonated | kWaiting
-    __shared__ unsigned long long sbusy[kSplit ? KP_TRACE_BLOCK / 64 : 1];  // wave: owners with helpers at work
+    LeafLds& leafl = S.leaf;
+    float4 (&wray)[2][KP_TRACE_BLOCK] = S.wray;
+    unsigned long long (&skey)[KP_TRACE_BLOCK] = S.split.key;
+    float4 (&shit)[KP_TRACE_BLOCK] = S.split.hit;
+    uint32_t (&srole)[KP_TRACE_BLOCK] = S.split.role;
+    unsigned long long (&sbusy)[KP_TRACE_BLOCK / 64] = S.split.busy;
     const int tid = threadIdx.x;
     const uint32_t gl = blockIdx.x * KP_TRACE_BLOCK + tid;
     Stack<kStack> st;
-    st.lds = lds;
+    st.lds = S.stack;
     st.spill = args.spill + (size_t)gl * args.spill_cap;
     st.cap = args.spill_cap;
     st.sp = 0;
@@ -682,9 +741,17 @@ __device__ __forceinline__ void traverse(const TraceArgs& args) {
     bool split_on = false;   // rays are being split (wave-uniform; roles live in srole)
     uint64_t cnt_nodes = 0, cnt_tris = 0;
     RayFeeder feed;
-    feed.init(args.counter, args.rays, args.roots, n_rays);
+    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks);
+    if (kConnect) {
+        set_open_count(leafl, tid, 0u);
+        __builtin_amdgcn_wave_barrier();
+    }
 
     for (;;) {
+        if (kConnect) {
+            const uint32_t open = open_count(leafl, tid);
+            if (open >= 64u) connect_open(args, leafl, open, tid);
+        }
         if (ray_id == KP_INVALID && feed.pid != KP_INVALID) {
             ray_id = feed.pid;
             setup_ray(feed.p0, feed.p1, r);
@@ -937,7 +1004,16 @@ __device__ __forceinline__ void traverse(const TraceArgs& args) {
                 }
                 if (done) {
                     const uint32_t role = kSplit && split_on ? srole[tid] : 0u;
-                    if (kAny) {
+                    if (kConnect) {
+                        const unsigned long long m = __ballot(!occl);
+                        if (!occl) {
+                            const uint32_t base = open_count(leafl, tid);
+                            leafl.open.ray[tid >> 6][base + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] =
+                                ray_id;
+                            __builtin_amdgcn_wave_barrier();
+                            set_open_count(leafl, tid, base + (uint32_t)__popcll(m));
+                        }
+                    } else if (kAny) {
                         args.occl[ray_id] = occl ? 1u : 0u;
                     } else if (kSplit && (role & kHelper)) {
                         // merge into the owner's slot: minimum key, then the
@@ -969,6 +1045,10 @@ __device__ __forceinline__ void traverse(const TraceArgs& args) {
             }
         }
     }
+    if (kConnect) {
+        const uint32_t open = open_count(leafl, tid);
+        if (open != 0u) connect_open(args, leafl, open, tid);
+    }
     if (kCount) {
         atomicAdd((unsigned long long*)&args.counters[0], (unsigned long long)cnt_nodes);
         atomicAdd((unsigned long long*)&args.counters[1], (unsigned long long)cnt_tris);
@@ -977,11 +1057,13 @@ __device__ __forceinline__ void traverse(const TraceArgs& args) {
 
 template <bool kCount>
 __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_closest(TraceArgs args) {
-    traverse<false, kCount, false>(args);
+    __shared__ TraceLds lds;
+    traverse<false, kCount, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_occluded(TraceArgs args) {
-    traverse<true, false, false>(args);
+    __shared__ TraceLds lds;
+    traverse<true, false, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
 // The same traversals compiled for 5 waves per SIMD (96 registers; closest
@@ -990,12 +1072,14 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_occluded(TraceArgs args) {
 // only the integrator launches them.
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_closest5(
     TraceArgs args) {
-    traverse<false, false, false>(args);
+    __shared__ TraceLds lds;
+    traverse<false, false, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_occluded5(
     TraceArgs args) {
-    traverse<true, false, false>(args);
+    __shared__ TraceLds lds;
+    traverse<true, false, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
 // The two-level traversals compiled for 5 waves per SIMD (96 registers, 44 B
@@ -1004,21 +1088,51 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
 // the 4-wave build.
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_closest_inst5(
     TraceArgs args) {
-    traverse<false, false, true>(args);
+    __shared__ TraceLds lds;
+    traverse<false, false, true>(args, lds, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_occluded_inst5(
     TraceArgs args) {
-    traverse<true, false, true>(args);
+    __shared__ TraceLds lds;
+    traverse<true, false, true>(args, lds, blockIdx.x, gridDim.x);
+}
+
+// A bounce's two traversals in one launch: blocks [0, n_closest) trace the
+// path rays (closest hit), the others the shadow rays of the vertices before
+// them (occlusion, connecting).  The two queues do not depend on each other,
+// and a persistent launch ends with a drain (its longest rays) in which the
+// machine empties: with both in one launch the shadow blocks start on every
+// CU as its closest-hit blocks run out, so a bounce has one drain, not two
+// (30 to 50 us each: most of a bounce of a small image).  The two-level build
+// spills 94 registers and is still faster than two launches: a two-level
+// terrain render 29.5 ms before, 27.4 now.
+template <bool kInst>
+__global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace_pair(
+    TraceArgs args, ShadowQueue q, uint32_t n_closest) {
+    __shared__ TraceLds lds;
+    if (blockIdx.x < n_closest) {
+        traverse<false, false, kInst>(args, lds, blockIdx.x, n_closest);
+    } else {
+        args.rays = q.rays;
+        args.n_dev = q.n_dev;
+        args.counter = q.counter;
+        args.roots = q.roots;
+        args.scontrib = q.contrib;
+        args.radiance = q.radiance;
+        traverse<true, false, kInst, true>(args, lds, blockIdx.x - n_closest, gridDim.x - n_closest);
+    }
 }
 
 template <bool kCount>
 __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_closest_inst(TraceArgs args) {
-    traverse<false, kCount, true>(args);
+    __shared__ TraceLds lds;
+    traverse<false, kCount, true>(args, lds, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_occluded_inst(TraceArgs args) {
-    traverse<true, false, true>(args);
+    __shared__ TraceLds lds;
+    traverse<true, false, true>(args, lds, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(256) void k_copy16(uint4* __restrict__ dst, const uint4* __restrict__ src,
@@ -1041,9 +1155,9 @@ __global__ void k_reset_u32(uint32_t* p, uint32_t n) {
 }
 
 // ---------------------------------------------------------------- launch --
-hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, hipStream_t s) {
+hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool reset, hipStream_t s) {
     if (grid == 0 || grid > a.spill_blocks) return hipErrorInvalidValue;   // lanes without a spill slice
-    hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
+    if (reset) hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
     if (a.insts) {
         if (count) hipLaunchKernelGGL(k_closest_inst<true>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
         else if (a.five_waves) hipLaunchKernelGGL(k_closest_inst5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
@@ -1063,6 +1177,16 @@ hipError_t launch_occluded(const TraceArgs& a, uint32_t grid, hipStream_t s) {
     else if (a.insts) hipLaunchKernelGGL(k_occluded_inst, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
     else if (a.five_waves) hipLaunchKernelGGL(k_occluded5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
     else hipLaunchKernelGGL(k_occluded, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair(const TraceArgs& a, const ShadowQueue& q, uint32_t grid_closest, uint32_t grid_occluded,
+                       hipStream_t s) {
+    if (grid_closest == 0 || grid_occluded == 0 || grid_closest + grid_occluded > a.spill_blocks)
+        return hipErrorInvalidValue;   // lanes without a spill slice
+    const dim3 grid(grid_closest + grid_occluded);
+    if (a.insts) hipLaunchKernelGGL(k_trace_pair<true>, grid, dim3(KP_TRACE_BLOCK), 0, s, a, q, grid_closest);
+    else hipLaunchKernelGGL(k_trace_pair<false>, grid, dim3(KP_TRACE_BLOCK), 0, s, a, q, grid_closest);
     return hipGetLastError();
 }
 

@@ -1,0 +1,52 @@
+"""The integrator's paired traversal launches (path rays and shadow rays of one
+bounce together, contributions added inside the traversal) at path counts
+around the wave, list and block sizes.  Path i of kp_integrate_rays draws
+from sequence i whatever the call's size, so n paths must equal the first n of
+a larger call bit for bit; the larger call is checked against the oracle path
+by path (2e-3 relative, the tolerance of the other per-path tests)."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from kazen_proto_amd import native, scenes
+
+pytestmark = pytest.mark.gpu
+CPU_THREADS = min(16, os.cpu_count() or 1)
+N_BIG = 3001
+
+
+def _scene(two_level):
+    if two_level:
+        return scenes.terrain_scene(grid=24, n_spheres=6, sphere_lon=12, sphere_lat=6, width=64, height=48,
+                                    max_depth=5, instanced=True)
+    return scenes.closures_scene(width=64, height=48, max_depth=5)
+
+
+@pytest.mark.parametrize("two_level", [False, True])
+@pytest.mark.parametrize("depth", [1, 5])
+def test_path_counts_around_the_edges(two_level, depth):
+    s = _scene(two_level)
+    s.max_depth = depth
+    c = native.Context(0)
+    c.load_scene(s, instances=native.INSTANCES_TWO_LEVEL if two_level else native.INSTANCES_AUTO)
+    rays = scenes.pinhole_rays(s.eye, s.lookat, s.up, s.fov_deg, s.width, s.height)[:N_BIG]
+    d = native.make_render_desc(s)
+    big = c.integrate_rays(rays, d)
+    st = c.render_stats()
+    od = oracle.RenderDesc()
+    od.width, od.height, od.spp = s.width, s.height, 1
+    od.max_depth, od.rr_depth, od.seed, od.spp_offset = s.max_depth, s.rr_depth, s.seed, 0
+    od.eye[:], od.lookat[:], od.up[:] = s.eye, s.lookat, s.up
+    od.tan_half_fov = s.tan_half_fov
+    ref = oracle.scene_from(s).integrate_rays(rays, od, threads=CPU_THREADS)
+    close = np.all(np.abs(big - ref) <= 2e-3 * np.abs(ref) + 1e-5, axis=1)
+    assert close.mean() >= 0.99
+    assert st["extension_rays"] >= N_BIG and 0 < st["shadow_rays"] <= st["extension_rays"]
+    for n in (1, 2, 63, 64, 65, 127, 129, 255, 256, 257, 1023, 2049):
+        part = c.integrate_rays(rays[:n], d)
+        assert np.array_equal(part.view(np.uint32), big[:n].view(np.uint32)), n
+    # a repeat gives the same bits
+    assert np.array_equal(c.integrate_rays(rays, d).view(np.uint32), big.view(np.uint32))
+    c.close()

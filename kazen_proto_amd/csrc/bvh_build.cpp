@@ -171,6 +171,22 @@ static uint16_t f16_int(uint32_t q) {
     return (uint16_t)(((uint32_t)(e + 15) << 10) | mant);
 }
 
+// Largest float <= v whose low byte is the exponent byte e.
+static float origin_below(float v, int8_t e) {
+    uint32_t b;
+    std::memcpy(&b, &v, 4);
+    const uint32_t byte = (uint8_t)e;
+    uint32_t c = (b & ~0xFFu) | byte;
+    if (b & 0x80000000u) {
+        if (c < b) c += 0x100u;          // negative: a larger magnitude is lower
+    } else if (c > b) {
+        c = b >= 0x100u ? c - 0x100u : 0x80000000u | byte;   // below the smallest positive: a negative one
+    }
+    float r;
+    std::memcpy(&r, &c, 4);
+    return r;
+}
+
 bool build_bvh8(const float* tris, uint32_t n_tris, const BuildOptions& opt, Bvh8Host& out,
                 std::string& err) {
     out = Bvh8Host{};
@@ -353,18 +369,25 @@ bool build_bvh8(const float* tris, uint32_t n_tris, const BuildOptions& opt, Bvh
         Box nb;
         for (uint32_t k : kids)
             if (k != kNoKid) nb.grow(b.nodes[k].box);
-        nd.px = nb.lo[0];
-        nd.py = nb.lo[1];
-        nd.pz = nb.lo[2];
+        float origin[3];
         int e[3];
         for (int k = 0; k < 3; ++k) {
             double ext = (double)nb.hi[k] - (double)nb.lo[k];
             int ek = -126;
             if (ext > 0.0) ek = (int)std::ceil(std::log2(ext / (double)kQMax));
             ek = std::max(-126, std::min(127, ek));
-            while (std::ldexp((double)kQMax, ek) < ext && ek < 127) ++ek;
+            // the origin carries the exponent in its low byte, so it lies up
+            // to 256 float steps below the box and the extent grows by that
+            for (;; ++ek) {
+                origin[k] = origin_below(nb.lo[k], (int8_t)ek);
+                ext = (double)nb.hi[k] - (double)origin[k];
+                if (std::ldexp((double)kQMax, ek) >= ext || ek >= 127) break;
+            }
             e[k] = ek;
         }
+        nd.px = origin[0];
+        nd.py = origin[1];
+        nd.pz = origin[2];
         nd.ex = (int8_t)e[0];
         nd.ey = (int8_t)e[1];
         nd.ez = (int8_t)e[2];

@@ -94,6 +94,15 @@ int trace_occluded_dev(kp_ctx* c, const float4* rays, uint32_t n, uint32_t* out)
     return KP_OK;
 }
 
+// Allocates c->d_nodes and uploads the device form of the node records.
+static int upload_nodes(kp_ctx* c, const std::vector<KpNode8>& nodes) {
+    std::vector<uint32_t> dev(32 * nodes.size());
+    for (size_t i = 0; i < nodes.size(); ++i) kp_device_node(nodes[i], &dev[32 * i]);
+    KP_HIP_TRY(c, hipMalloc((void**)&c->d_nodes, dev.size() * 4));
+    KP_HIP_TRY(c, hipMemcpy(c->d_nodes, dev.data(), dev.size() * 4, hipMemcpyHostToDevice));
+    return KP_OK;
+}
+
 static void free_bvh(kp_ctx* c) {
     c->host = HostBvh();
     if (c->d_nodes) (void)hipFree(c->d_nodes);
@@ -292,12 +301,12 @@ static int build_two_level(kp_ctx* c, const BuildOptions& bo, double* seconds) {
     // Postponed leaves need no stack entries.
     c->spill_cap = 8u * top.max_depth + 7u * max_unit_depth + 16u;
     if (c->device >= 0) {
-        const size_t nb = nodes.size() * sizeof(KpNode8), tbytes = tris.size() * sizeof(float);
-        KP_HIP_TRY(c, hipMalloc((void**)&c->d_nodes, nb));
+        const size_t tbytes = tris.size() * sizeof(float);
+        const int urc = upload_nodes(c, nodes);
+        if (urc) return urc;
         KP_HIP_TRY(c, hipMalloc((void**)&c->d_tris, tbytes));
         KP_HIP_TRY(c, hipMalloc((void**)&c->d_insts, rec.size() * sizeof(float)));
         KP_HIP_TRY(c, hipMalloc((void**)&c->d_tlas_inst, top.tri_order.size() * 4));
-        KP_HIP_TRY(c, hipMemcpy(c->d_nodes, nodes.data(), nb, hipMemcpyHostToDevice));
         KP_HIP_TRY(c, hipMemcpy(c->d_tris, tris.data(), tbytes, hipMemcpyHostToDevice));
         KP_HIP_TRY(c, hipMemcpy(c->d_insts, rec.data(), rec.size() * sizeof(float), hipMemcpyHostToDevice));
         KP_HIP_TRY(c, hipMemcpy(c->d_tlas_inst, top.tri_order.data(), top.tri_order.size() * 4,
@@ -651,10 +660,10 @@ static int install_one_level(kp_ctx* c, kp::Bvh8Host& h, uint32_t n_all, uint32_
     // top KP_TRACE_STACK entries live in LDS.
     c->spill_cap = 7u * h.max_depth + 8u;
     if (c->device >= 0) {
-        const size_t nb = h.nodes.size() * sizeof(KpNode8), tb = h.tris.size() * sizeof(float);
-        KP_HIP_TRY(c, hipMalloc((void**)&c->d_nodes, nb));
+        const size_t tb = h.tris.size() * sizeof(float);
+        const int urc = kp::upload_nodes(c, h.nodes);
+        if (urc) return urc;
         KP_HIP_TRY(c, hipMalloc((void**)&c->d_tris, tb));
-        KP_HIP_TRY(c, hipMemcpy(c->d_nodes, h.nodes.data(), nb, hipMemcpyHostToDevice));
         KP_HIP_TRY(c, hipMemcpy(c->d_tris, h.tris.data(), tb, hipMemcpyHostToDevice));
         c->spill_lanes = (size_t)kp::max_trace_grid(c) * KP_TRACE_BLOCK;
         KP_HIP_TRY(c, hipMalloc((void**)&c->d_spill, c->spill_lanes * c->spill_cap * sizeof(uint2)));

@@ -349,10 +349,10 @@ __global__ void k_pass_advance(unsigned long long* pass, uint32_t paths) {
 __global__ void k_rebase_nodes(uint4* nodes, uint32_t n, uint32_t node_off, uint32_t tri_off) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    uint4 w = nodes[8 * (size_t)i + 1];   // dwords 4-7: child_base, prim_base, meta
-    w.x += node_off;
-    w.y += tri_off;
-    nodes[8 * (size_t)i + 1] = w;
+    // dword 3: child_base (24 bits; the batch holds fewer than 2^24 nodes) | imask; dword 4: prim_base
+    uint32_t* w = reinterpret_cast<uint32_t*>(nodes + 8 * (size_t)i);
+    w[3] = ((w[3] + node_off) & 0x00FFFFFFu) | (w[3] & 0xFF000000u);
+    w[4] += tri_off;
 }
 __global__ void k_rebase_tris(float4* tris, uint32_t n, uint32_t prim_off) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;

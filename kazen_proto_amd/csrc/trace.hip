@@ -12,10 +12,10 @@
 //    prefix count), so incoherent rays do not leave idle lanes behind;
 //  - a per-lane short stack in LDS (kStack group entries); deeper entries
 //    spill to a per-lane region in HBM, so any BVH depth works;
-//  - 128-byte nodes: eight 16-byte loads per visit (each lane loads its own
-//    near and far planes by the ray's octant), 16-bit child boxes decoded
-//    with one fma per plane; hit leaves are tested at once, the nearest hit
-//    inner child is visited next and the others go on the stack as one group,
+//  - 128-byte nodes: seven 16-byte loads per visit (each lane loads its own
+//    near and far planes by the ray's octant; the leaf words are read only
+//    when leaf children are tested), 16-bit child boxes decoded with one fma
+//    per plane; the nearest hit inner child is visited next and the others go on the stack as one group,
 //    visited in octant order (children sit in octant slots) and culled as a
 //    group by their nearest entry distance;
 //  - watertight ray/triangle test (Woop, Benthin, Wald 2013) with contraction
@@ -185,36 +185,50 @@ __device__ __forceinline__ float qplane(const uint4& plane, int slot) {
 
 // Result of one node visit.
 struct NodeHits {
-    uint4 w0, w1;        // header words (origin / exponents / inner mask, bases / meta)
+    uint32_t group;      // first inner child | inner mask << 24
     uint32_t inner;      // inner children hit (slot bits)
     uint32_t leaves;     // leaf children hit (slot bits)
-    uint32_t near_key;   // (tnear key | slot) of the nearest inner child hit
-    uint32_t next_key;   // the same for the second nearest (0xFFFFFFFF if none)
+    int32_t near_key;    // (tnear key | slot) of the nearest inner child hit
+    int32_t next_key;    // the same for the second nearest (kNoKey if none)
 };
 
-// Order key of a child entry distance: non-negative distances by their bits
-// (monotone), negative ones (sign bit set: negative as integers) all first.
-__device__ __forceinline__ uint32_t tkey(float tn) {
-    return (uint32_t)max((int32_t)__float_as_uint(tn), 0) & 0xFFFFFFF8u;
+// Order key of a child entry distance, as a signed integer: non-negative
+// distances by their bits (monotone), negative ones (sign bit set: negative
+// as integers) all first.
+constexpr int32_t kNoKey = 0x7FFFFFFF;
+__device__ __forceinline__ int32_t tkey(float tn, uint32_t slot) {
+    return (int32_t)((__float_as_uint(tn) & 0xFFFFFFF8u) | slot);
 }
 
-// Tests the 8 children of node `idx` against [tmin, tmax].
+// (the compiler does not form it from min and max here)
+__device__ __forceinline__ int32_t median3(int32_t a, int32_t b, int32_t c) {
+    int32_t m;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+}
+
+// Tests the 8 children of node `idx` against [tmin, tmax].  Measured on the
+// 4.2 M incoherent rays (1,148,576 triangles): the vector ALU issues in 89 %
+// of its cycles and the L1's data return is busy in 89 % of its own, so a
+// visit's instructions and its loads both cost time.  With seven loads (leaf
+// words only where leaves are tested), signed order keys (no clamp at zero),
+// the running second minimum as a median, and the hit kept in LDS instead of
+// four registers: 1,284 -> 1,188 us a launch.
 __device__ __forceinline__ void visit_node(NodeBuf nb, uint32_t idx, const RayPre& r, const NodeTest& nt,
                                            float tmax, NodeHits& h) {
     const uint32_t p = idx << 7;   // 128-byte nodes
-    h.w0 = node_word(nb, p);
-    h.w1 = node_word(nb, p + 16u);
+    const uint4 w0 = node_word(nb, p);
     const uint4 nx = node_word(nb, p + (nt.offa & 0xFFu)), fx = node_word(nb, p + ((nt.offa >> 8) & 0xFFu));
     const uint4 ny = node_word(nb, p + ((nt.offa >> 16) & 0xFFu)), fy = node_word(nb, p + (nt.offa >> 24));
     const uint4 nz = node_word(nb, p + (nt.offb & 0xFFu)), fz = node_word(nb, p + (nt.offb >> 8));
-    const float px = __uint_as_float(h.w0.x), py = __uint_as_float(h.w0.y), pz = __uint_as_float(h.w0.z);
-    const uint32_t e = h.w0.w;
-    const int ex = (int)(int8_t)(e & 0xFF), ey = (int)(int8_t)((e >> 8) & 0xFF), ez = (int)(int8_t)((e >> 16) & 0xFF);
+    const float px = __uint_as_float(w0.x), py = __uint_as_float(w0.y), pz = __uint_as_float(w0.z);
+    const int ex = (int)(int8_t)(w0.x & 0xFF), ey = (int)(int8_t)(w0.y & 0xFF), ez = (int)(int8_t)(w0.z & 0xFF);
     // ix 2^ex: a product with a power of two, exact as the multiplication
     const float ax = ldexpf(r.ix, ex), ay = ldexpf(r.iy, ey), az = ldexpf(r.iz, ez);
     const float bx = (px - r.ox) * r.ix, by = (py - r.oy) * r.iy, bz = (pz - r.oz) * r.iz;
-    const uint32_t imask = e >> 24;
-    uint32_t hit = 0u, k1 = 0xFFFFFFFFu, k2 = 0xFFFFFFFFu;
+    const uint32_t imask = w0.w >> 24;
+    uint32_t hit = 0u;
+    int32_t k1 = kNoKey, k2 = kNoKey;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
         const float tnx = fmaf(qplane(nx, s), ax, bx);
@@ -227,14 +241,16 @@ __device__ __forceinline__ void visit_node(NodeBuf nb, uint32_t idx, const RayPr
         const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
         const bool hs = tn <= fmaf(fabsf(tf), KP_FAR_EPS, tf);
         hit |= hs ? (1u << s) : 0u;
-        // key of a hit inner child: entry distance bits (non-positive -> 0), slot
-        const uint32_t key = (hs && ((imask >> s) & 1u)) ? (tkey(tn) | (uint32_t)s) : 0xFFFFFFFFu;
-        k2 = min(k2, max(k1, key));
+        // key of a hit inner child; k1 <= k2, so the second smallest of
+        // {k1, k2, key} is their median
+        const int32_t key = (hs && ((imask >> s) & 1u)) ? tkey(tn, (uint32_t)s) : kNoKey;
+        k2 = median3(k1, k2, key);
         k1 = min(k1, key);
     }
     // Empty slots hold inverted boxes (lower plane 2047, upper plane 0), which
     // miss unless the far-distance widening exceeds the node's extent; such a
     // slot then counts as a leaf child with no triangles and tests nothing.
+    h.group = w0.w;
     h.inner = hit & imask;
     h.leaves = hit & ~imask;
     h.near_key = k1;
@@ -258,9 +274,8 @@ __device__ __forceinline__ uint32_t oct_permute(uint32_t m, uint32_t oct) {
 //   y = lower bound of the group's entry distances (float bits, low 8 bits
 //       cleared: a truncation toward zero, or -inf) | remaining children as
 //       octant-rank bits (8 bits).
-__device__ __forceinline__ uint32_t group_bound_bits(uint32_t key2) {
-    if (key2 == 0xFFFFFFFFu || key2 < 8u) return 0xFF800000u;   // none, or a negative distance: -inf
-    return key2 & 0xFFFFFF00u;
+__device__ __forceinline__ uint32_t group_bound_bits(int32_t key2) {
+    return key2 < 0 ? 0xFF800000u : (uint32_t)key2 & 0xFFFFFF00u;   // a negative distance: -inf
 }
 
 // Entry distance of one child slot of node `idx` (the same arithmetic as
@@ -270,8 +285,7 @@ __device__ __forceinline__ float slot_tnear(const uint4* __restrict__ nodes, uin
     const uint4* p = nodes + (size_t)idx * 8;
     const uint4 w0 = p[0];
     const uint4 nx = p[(nt.offa & 0xFFu) >> 4], ny = p[((nt.offa >> 16) & 0xFFu) >> 4], nz = p[(nt.offb & 0xFFu) >> 4];
-    const uint32_t e = w0.w;
-    const int ex = (int)(int8_t)(e & 0xFF), ey = (int)(int8_t)((e >> 8) & 0xFF), ez = (int)(int8_t)((e >> 16) & 0xFF);
+    const int ex = (int)(int8_t)(w0.x & 0xFF), ey = (int)(int8_t)(w0.y & 0xFF), ez = (int)(int8_t)(w0.z & 0xFF);
     const float ax = ldexpf(r.ix, ex), ay = ldexpf(r.iy, ey), az = ldexpf(r.iz, ez);
     const float bx = (__uint_as_float(w0.x) - r.ox) * r.ix, by = (__uint_as_float(w0.y) - r.oy) * r.iy,
                 bz = (__uint_as_float(w0.z) - r.oz) * r.iz;
@@ -328,6 +342,10 @@ struct Stack {
         lds[sp & (S - 1)][tid] = make_uint2(a, b);
         ++sp;
         return true;
+    }
+    __device__ __forceinline__ void push_lds(uint32_t a, uint32_t b) {   // sp < S
+        lds[sp][tid] = make_uint2(a, b);
+        ++sp;
     }
     __device__ __forceinline__ uint2 top() const { return lds[(sp - 1) & (S - 1)][tid]; }
     __device__ __forceinline__ void set_top_y(uint32_t y) { lds[(sp - 1) & (S - 1)][tid].y = y; }
@@ -446,7 +464,8 @@ constexpr uint32_t kStuckBatch = 8u;
 // per lane, the merged result of the triangles tested for its ray.
 struct LeafLds {
     uint32_t map[KP_TRACE_BLOCK];             // wave's 64 entries: owner lane << 8 | item of the owner
-    unsigned long long key[KP_TRACE_BLOCK];   // closest hit: minimum hit key; any hit: nonzero once hit
+    unsigned long long key[KP_TRACE_BLOCK];   // closest hit: minimum hit key of the lane's ray, ~0 if none;
+                                              // any hit: nonzero once hit
     union {
         float4 hit[KP_TRACE_BLOCK];           // closest hit: {t, u, v} of the minimum key
         struct {                              // any hit, connecting: rays found unoccluded
@@ -458,10 +477,18 @@ struct LeafLds {
 
 __device__ __forceinline__ unsigned long long hit_key(float t, uint32_t prim);
 
+// A closest-hit lane reads the leaf words of a set when the wave tests it, an
+// occlusion lane when it finds the set (three registers more; the closest-hit
+// builds have none to spare: with the words in registers they spill in the
+// loop and the 4.2 M incoherent rays take 1,272 us instead of 1,228).
+template <bool kAny>
+constexpr bool kLazyLeaves = !kAny;
+
 // Tests the postponed leaf sets of all active lanes of the wave together.
-// Each lane holds up to two sets (leaf slots `pend` of a node with primitive
-// base `pbase` and meta words m0 / m1: per slot first offset and count; the
-// second set is the one found in the current iteration); a lane's sets are
+// Each lane holds up to two sets (node << 8 | its hit leaf slots, 0 if none;
+// the node's leaf words, primitive base and per slot first offset and count,
+// are read here; the second set is the one found in the current iteration); a
+// lane's sets are
 // one run of triangle tests (at most 2 x 8 slots x 4 = 64); the runs are laid
 // out as one list (exclusive prefix sums over the lanes) and dealt out to the
 // active lanes, as many as there are per round, so the triangle tests run with nearly every lane busy instead of
@@ -469,9 +496,11 @@ __device__ __forceinline__ unsigned long long hit_key(float t, uint32_t prim);
 // owner's ray and closest distance from the owner's registers (lane
 // permutes) and merges a hit into the owner's LDS slot: the 64-bit minimum of
 // the (distance, primitive) key, then the t, u, v of the lane whose key is
-// the minimum.  Every triangle is tested against the owner's closest distance
-// at the start of the batch, so the owner's new closest hit is the minimum
-// key over its hits, the same as testing them one after another.
+// the minimum.  The slot lasts as long as the ray (key ~0: no hit yet), so a
+// lane keeps only its closest distance in a register.  Every triangle is
+// tested against the owner's closest distance at the start of the batch, so
+// the slot holds the minimum key over all hits, the same as testing them one
+// after another.
 __device__ __forceinline__ uint32_t leaf_set_tris(uint32_t pend, uint32_t m0, uint32_t m1) {
     // slot bits of pend spread to byte masks (bit k -> byte k), then a byte sum
     const uint32_t b0 = (((pend & 0xFu) * 0x00204081u) & 0x01010101u) * 0xFFu;
@@ -481,11 +510,14 @@ __device__ __forceinline__ uint32_t leaf_set_tris(uint32_t pend, uint32_t m0, ui
 }
 
 template <bool kAny, bool kCount>
-__device__ __forceinline__ void test_leaves_wave(const float4* __restrict__ tris, const RayPre& r, uint32_t pend,
-                                                 uint32_t pbase, uint32_t m0, uint32_t m1, uint32_t pend2,
-                                                 uint32_t pbase2, uint32_t m02, uint32_t m12, float& best_t,
-                                                 uint32_t& best_p, float& bu, float& bv, bool& occl,
+__device__ __forceinline__ void test_leaves_wave(NodeBuf nb, const float4* __restrict__ tris, const RayPre& r,
+                                                 uint32_t set1, const uint4& pw, uint32_t set2, float& best_t, bool& occl,
                                                  uint64_t& cnt_tris, uint32_t prim_off, LeafLds& L, int tid) {
+    const uint32_t pend = set1 & 0xFFu, pend2 = set2 & 0xFFu;
+    uint4 w1 = pw, w2 = make_uint4(0u, 0u, 0u, 0u);
+    if (kLazyLeaves<kAny> && pend) w1 = node_word(nb, ((set1 >> 8) << 7) + 16u);
+    if (pend2) w2 = node_word(nb, ((set2 >> 8) << 7) + 16u);
+    const uint32_t pbase = w1.x, m0 = w1.y, m1 = w1.z, pbase2 = w2.x, m02 = w2.y, m12 = w2.z;
     const uint32_t lane = __lane_id();
     const unsigned long long below = (1ull << lane) - 1ull;
     const unsigned long long active = __ballot(true);
@@ -507,7 +539,7 @@ __device__ __forceinline__ void test_leaves_wave(const float4* __restrict__ tris
     if (P == 0u) return;
     const int wbase = tid & ~63;
     uint32_t* map = &L.map[wbase];
-    if (T != 0u) L.key[tid] = kAny ? 0ull : ~0ull;
+    if (kAny && T != 0u) L.key[tid] = 0ull;
     for (uint32_t base = 0u; base < P; base += nact) {
         if (T != 0u) {
             const uint32_t lo = max(E, base), hi = min(E + T, base + nact);
@@ -563,6 +595,7 @@ __device__ __forceinline__ void test_leaves_wave(const float4* __restrict__ tris
                     L.key[ot] = 1ull;
                 } else {
                     const unsigned long long hk = hit_key(t, __float_as_uint(ta.w) + o_off);
+                    // (no other triangle of the ray has this key)
                     __hip_atomic_fetch_min(&L.key[ot], hk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
                     __builtin_amdgcn_wave_barrier();
                     if (__hip_atomic_load(&L.key[ot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) == hk)
@@ -576,12 +609,8 @@ __device__ __forceinline__ void test_leaves_wave(const float4* __restrict__ tris
         const unsigned long long k = __hip_atomic_load(&L.key[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
         if (kAny) {
             if (k != 0ull) occl = true;
-        } else if (k != ~0ull && (best_p == KP_INVALID || k < hit_key(best_t, best_p))) {
-            const float4 h = L.hit[tid];
-            best_t = h.x;
-            best_p = (uint32_t)k;
-            bu = h.y;
-            bv = h.z;
+        } else if (k != ~0ull) {
+            best_t = L.hit[tid].x;
         }
     }
 }
@@ -595,6 +624,13 @@ __device__ __forceinline__ unsigned long long hit_key(float t, uint32_t prim) {
     if (b == 0x80000000u) b = 0u;
     b ^= (b & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u;
     return ((unsigned long long)b << 32) | prim;
+}
+
+// Writes a ray's hit record from its slot's key and {t, u, v}.
+__device__ __forceinline__ void write_hit(float4* out, unsigned long long key, const float4& h) {
+    const bool none = key == ~0ull;
+    *out = none ? make_float4(__int_as_float(0x7f800000), __uint_as_float(KP_INVALID), 0.0f, 0.0f)
+                : make_float4(h.x, __uint_as_float((uint32_t)key), h.y, h.z);
 }
 
 // Position of the set bit of rank r (0-based) in m; r < popcount(m).
@@ -733,9 +769,10 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
     uint32_t ray_id = KP_INVALID;
     RayPre r;
     NodeTest nt;
-    float best_t = 0.0f, bu = 0.0f, bv = 0.0f;
-    uint32_t best_p = KP_INVALID, cur = KP_INVALID, steps = 0;
-    uint32_t pend = 0u, pbase = 0u, pm0 = 0u, pm1 = 0u;   // postponed leaf children
+    float best_t = 0.0f;                                   // closest distance so far (the hit itself is in LDS)
+    uint32_t cur = KP_INVALID, steps = 0;
+    uint32_t pend = 0u;                                    // postponed leaf children: node << 8 | slots
+    uint4 pw = make_uint4(0u, 0u, 0u, 0u);                 // the leaf words of that node (!kLazyLeaves)
     uint32_t inst_pbase = 0u;                              // primitive base of the instance entered
     bool occl = false;
     bool split_on = false;   // rays are being split (wave-uniform; roles live in srole)
@@ -757,8 +794,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
             setup_ray(feed.p0, feed.p1, r);
             nt = node_test_setup(r);
             best_t = r.tmax;
-            best_p = KP_INVALID;
-            bu = bv = 0.0f;
+            if (!kAny) leafl.key[tid] = ~0ull;
             occl = false;
             pend = 0u;
             inst_pbase = 0u;
@@ -799,18 +835,8 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 __builtin_amdgcn_wave_barrier();
                 const unsigned long long busy = __hip_atomic_load(busy_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
                 if (ray_id != KP_INVALID && (role & kWaiting) && !((busy >> lane) & 1ull)) {
-                    const unsigned long long k = skey[tid];
-                    if (k != ~0ull && (best_p == KP_INVALID || k < hit_key(best_t, best_p))) {
-                        const float4 h = shit[tid];
-                        best_t = h.x;
-                        best_p = (uint32_t)k;
-                        bu = h.y;
-                        bv = h.z;
-                    }
-                    float4 hh;
-                    if (best_p == KP_INVALID) hh = make_float4(__int_as_float(0x7f800000), __uint_as_float(KP_INVALID), 0.0f, 0.0f);
-                    else hh = make_float4(best_t, __uint_as_float(best_p), bu, bv);
-                    args.hits[ray_id] = hh;
+                    const unsigned long long k = skey[tid], own = leafl.key[tid];
+                    write_hit(args.hits + ray_id, k < own ? k : own, k < own ? shit[tid] : leafl.hit[tid]);
                     ray_id = KP_INVALID;
                 }
             }
@@ -820,7 +846,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 const float ob = __shfl(best_t, (int)(role & 63u));
                 if (ray_id != KP_INVALID && (role & kHelper) && ob < best_t) {
                     best_t = ob;
-                    best_p = KP_INVALID;
+                    leafl.key[tid] = ~0ull;
                 }
             }
             // idle lanes take the top group entry of lanes still at work
@@ -852,8 +878,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                         setup_ray(args.rays[2 * (size_t)rid], args.rays[2 * (size_t)rid + 1], r);
                         nt = node_test_setup(r);
                         best_t = bt;
-                        best_p = KP_INVALID;
-                        bu = bv = 0.0f;
+                        leafl.key[tid] = ~0ull;
                         pend = 0u;
                         cur = KP_INVALID;
                         steps = 0;
@@ -868,7 +893,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
         if (ray_id != KP_INVALID && steps != kStepsWaiting) {
             for (;;) {
                 bool fault = false;
-                uint32_t pend2 = 0u, pbase2 = 0u, pm02 = 0u, pm12 = 0u;   // a second leaf set found this iteration
+                uint32_t pend2 = 0u;   // a second leaf set found this iteration
                 if (cur != KP_INVALID) {
                     NodeHits h;
                     visit_node(nbuf, cur, r, nt, best_t, h);
@@ -878,13 +903,14 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                     if (kInst && h.leaves && vis < args.n_tlas) {
                         // top-level leaves: push every instance they name
                         uint32_t lm = h.leaves;
+                        const uint4 w1 = node_word(nbuf, (vis << 7) + 16u);
                         while (lm && !fault) {
                             const uint32_t s = __ffs(lm) - 1u;
                             lm &= lm - 1u;
-                            const uint32_t mw = s < 4u ? h.w1.z : h.w1.w;
+                            const uint32_t mw = s < 4u ? w1.y : w1.z;
                             const uint32_t meta = (mw >> ((s & 3u) * 8u)) & 0xFFu;
-                            const uint32_t first = h.w1.y + (meta & 31u), count = meta >> 5;
-                            const uint32_t gy = group_bound_bits(tkey(slot_tnear(nodes, vis, s, r, nt)));
+                            const uint32_t first = w1.x + (meta & 31u), count = meta >> 5;
+                            const uint32_t gy = group_bound_bits(tkey(slot_tnear(nodes, vis, s, r, nt), 0u));
                             for (uint32_t i = 0; i < count; ++i) {
                                 if (!st.push(args.tlas_inst[first + i], gy)) {
                                     atomicOr(args.err, 1u);
@@ -894,31 +920,28 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                             }
                         }
                     } else if (h.leaves) {
+                        // (the words' load is waited for with the next visit's)
+                        const uint32_t set = (vis << 8) | h.leaves;
                         if (pend == 0u) {
-                            pend = h.leaves;
-                            pbase = h.w1.y;
-                            pm0 = h.w1.z;
-                            pm1 = h.w1.w;
-                        } else {   // this lane already holds a set: the wave tests it below
-                            pend2 = h.leaves;
-                            pbase2 = h.w1.y;
-                            pm02 = h.w1.z;
-                            pm12 = h.w1.w;
+                            pend = set;
+                            if (!kLazyLeaves<kAny>) pw = node_word(nbuf, (vis << 7) + 16u);
+                        } else {   // this lane already holds a set: the wave tests both below
+                            pend2 = set;
                         }
                     }
                     if (h.inner && !fault && !(kAny && occl)) {
-                        const uint32_t imask = h.w0.w >> 24;
-                        const uint32_t s1 = h.near_key & 7u;
+                        const uint32_t s1 = (uint32_t)h.near_key & 7u;
                         const uint32_t rest = h.inner & ~(1u << s1);
                         if (rest) {
-                            const uint32_t gx = (h.w1.x & 0x00FFFFFFu) | (imask << 24);
                             const uint32_t gy = group_bound_bits(h.next_key) | oct_permute(rest, nt.oct);
-                            if (!st.push(gx, gy)) {
+                            if (__ballot(st.sp >= kStack) == 0ull) {   // nearly always: no lane spills
+                                st.push_lds(h.group, gy);
+                            } else if (!st.push(h.group, gy)) {
                                 atomicOr(args.err, 1u);
                                 fault = true;
                             }
                         }
-                        cur = inner_child(h.w1.x, imask, s1);
+                        cur = inner_child(h.group & 0x00FFFFFFu, h.group >> 24, s1);
                     }
                 }
                 if (!fault && cur == KP_INVALID && !(kAny && occl)) {
@@ -993,8 +1016,8 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 const uint32_t n_here = (uint32_t)__popcll(__ballot(true));
                 if (n_stuck >= min(kStuckBatch, n_here) || __ballot(pend2 != 0u) != 0ull ||
                     __popcll(__ballot(pend != 0u)) >= kLeafBatch) {
-                    test_leaves_wave<kAny, kCount>(tris, r, pend, pbase, pm0, pm1, pend2, pbase2, pm02, pm12, best_t,
-                                                   best_p, bu, bv, occl, cnt_tris, inst_pbase, leafl, tid);
+                    test_leaves_wave<kAny, kCount>(nbuf, tris, r, pend, pw, pend2, best_t, occl, cnt_tris, inst_pbase,
+                                                   leafl, tid);
                     pend = 0u;
                 }
                 bool done = fault || (kAny && occl) || (cur == KP_INVALID && pend == 0u && st.sp == 0);
@@ -1019,12 +1042,12 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                         // merge into the owner's slot: minimum key, then the
                         // t, u, v of the lane whose key is the minimum
                         const uint32_t o = role & 0xFFu;
-                        if (best_p != KP_INVALID) {
-                            const unsigned long long k = hit_key(best_t, best_p);
+                        const unsigned long long k = leafl.key[tid];
+                        if (k != ~0ull) {
                             __hip_atomic_fetch_min(&skey[o], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
                             __builtin_amdgcn_wave_barrier();
                             if (__hip_atomic_load(&skey[o], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) == k)
-                                shit[o] = make_float4(best_t, bu, bv, 0.0f);
+                                shit[o] = leafl.hit[tid];
                         }
                     } else if (kSplit && (role & kDonated)) {
                         srole[tid] = role | kWaiting;   // the hit is written once the helpers are done
@@ -1032,10 +1055,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                         pend = 0u;
                         break;
                     } else {
-                        float4 hh;
-                        if (best_p == KP_INVALID) hh = make_float4(__int_as_float(0x7f800000), __uint_as_float(KP_INVALID), 0.0f, 0.0f);
-                        else hh = make_float4(best_t, __uint_as_float(best_p), bu, bv);
-                        args.hits[ray_id] = hh;
+                        write_hit(args.hits + ray_id, leafl.key[tid], leafl.hit[tid]);
                     }
                     ray_id = KP_INVALID;
                     pend = 0u;

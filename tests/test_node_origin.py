@@ -1,0 +1,69 @@
+"""The builder's node origins carry the axis exponent in their low byte (the
+device node's header has no exponent word of its own): the property itself,
+and that boxes stay conservative where the low byte moves the origin most
+(origins at zero, negative, far from zero, tiny extents).  Closest hits over
+such trees equal brute force bit for bit."""
+import numpy as np
+import pytest
+
+import oracle
+from kazen_proto_amd import native, scenes
+
+CASES = [(0.0, 1.0), (-3.0, 1.0), (1.0e4, 1.0), (0.0, 1.0e-6), (5.0, 1.0e-4), (-1.0e3, 1.0e3)]
+
+
+def _tris(offset, scale, positive):
+    rng = np.random.default_rng(7)
+    c = rng.uniform(0.0 if positive else -1.0, 1.0, (700, 1, 3))
+    v = c + rng.normal(scale=0.05, size=(700, 3, 3))
+    if positive:
+        v = np.abs(v)
+        v[:50, :, 1] = 0.0                     # a flat patch through the origin's plane
+    return (v * scale + offset).reshape(-1, 9).astype(np.float32)
+
+
+@pytest.mark.parametrize("positive", [False, True])
+@pytest.mark.parametrize("offset,scale", CASES)
+def test_origin_low_byte_and_conservative_boxes(offset, scale, positive):
+    tris = _tris(offset, scale, positive)
+    nodes, t12, _ = native.bvh8_build_host(tris)
+    n = nodes.reshape(-1, 128)
+    assert np.array_equal(n[:, [0, 4, 8]], n[:, 12:15])          # low bytes of px, py, pz = ex, ey, ez
+    p = n[:, 0:12].copy().view(np.float32).astype(np.float64)
+    e = n[:, 12:15].view(np.int8).astype(np.int32)
+    q = n[:, 32:128].copy().view(np.float16).reshape(-1, 6, 8).astype(np.float64)
+    sc = np.ldexp(1.0, e)
+    v = t12.reshape(-1, 12)[:, [0, 1, 2, 4, 5, 6, 8, 9, 10]].reshape(-1, 3, 3).astype(np.float64)
+    base = n[:, 20:24].copy().view(np.uint32)[:, 0]
+    for i in range(n.shape[0]):
+        for s in range(8):
+            m = int(n[i, 24 + s])
+            if m == 0 or (n[i, 15] >> s) & 1:
+                continue
+            first = int(base[i]) + (m & 31)
+            pts = v[first:first + (m >> 5)].reshape(-1, 3)
+            assert np.all(pts >= p[i] + q[i, 0:3, s] * sc[i]) and np.all(pts <= p[i] + q[i, 3:6, s] * sc[i])
+    rng = np.random.default_rng(8)
+    rays = scenes.incoherent_rays(600, rng)
+    rays[:, 0:3] = rays[:, 0:3] * scale + offset
+    got = native.HostBvh8(tris).closest(rays)
+    assert np.array_equal(got.view(np.uint32), oracle.closest_bruteforce(tris, rays).view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset,scale", CASES)
+def test_device_nodes_give_the_same_hits(offset, scale):
+    tris = _tris(offset, scale, True)
+    rng = np.random.default_rng(9)
+    rays = scenes.incoherent_rays(4097, rng)
+    rays[:, 0:3] = rays[:, 0:3] * scale + offset
+    rays[::5, 3] = -0.3 * scale                # negative interval starts
+    rays[1::7, 7] = 0.4 * scale
+    c = native.Context(0)
+    c.mesh_add_soup(tris)
+    c.bvh_build()
+    ref = oracle.closest_bruteforce(tris, rays)
+    assert np.array_equal(c.intersect_closest(rays).view(np.uint32), ref.view(np.uint32))
+    want = oracle.closest_bruteforce(tris, rays)[:, 1].view(np.uint32) != 0xFFFFFFFF
+    assert np.array_equal(c.occluded(rays) != 0, want)
+    c.close()

@@ -367,6 +367,9 @@ constexpr int kStack = KP_TRACE_STACK;
 // memory round trip.  All members except the prefetch are wave-uniform.
 constexpr uint32_t kChunk = 256;
 constexpr uint32_t kTailChunk = 64;
+// Occlusion launches of at most this many rays per block split their rays
+// (k_occluded5<true>).
+constexpr uint32_t kSplitRays = 256;
 
 struct RayFeeder {
     uint32_t next, end, n;
@@ -381,7 +384,7 @@ struct RayFeeder {
 
     // block / blocks: this block's index among the blocks that share the queue
     __device__ __forceinline__ void init(uint32_t* ctr, const float4* rs, const uint32_t* rts, uint32_t count,
-                                         uint32_t block, uint32_t blocks) {
+                                         uint32_t block, uint32_t blocks, bool thin) {
         counter = ctr;
         rays = rs;
         roots = rts;
@@ -394,14 +397,23 @@ struct RayFeeder {
         // and a wave whose first chunk lies beyond the rays has none.
         waves = blocks * (KP_TRACE_BLOCK / 64);
         const uint32_t wave = block * (KP_TRACE_BLOCK / 64) + (threadIdx.x >> 6);
-        // up to kChunk rays per wave: every ray in a first chunk (multiples of
-        // 64, as many waves as that takes); more: the first chunks hold
-        // about half the rays (256 .. 4096 per wave) and the counter's chunks
-        // balance the rest
+        // up to kChunk rays per wave: every ray in a first chunk; more: the
+        // first chunks hold about half the rays (256 .. 4096 per wave) and the
+        // counter's chunks balance the rest.  First chunks are multiples of 64
+        // rays (as many waves as that takes), except that a small launch whose
+        // rays can be split (thin) uses one wave per SIMD with fewer rays each
+        // (a grid holds five): the idle lanes then take parts of the rays from
+        // the start.  1,000 / 16,384 closest-hit rays 45 / 97 us with 64 a
+        // wave, 35 / 75 so (with every wave used 65,536 rays take 57 us where
+        // three launches are in flight, 40 so).  Occlusion rays end early and
+        // lose by it (2,000 rays 71 -> 77 us).
         uint32_t first;
-        if (n <= waves * kChunk) {
+        const uint32_t per_simd = waves >= 5u ? waves / 5u : 1u;
+        if (thin && n <= per_simd * 64u) {
+            first = (n + per_simd - 1u) / per_simd;
+            first = first < 4u ? 4u : first;
+        } else if (n <= waves * kChunk) {
             first = ((n + waves - 1u) / waves + 63u) & ~63u;
-            if (first == 0u) first = 64u;
         } else {
             first = (n / (2u * waves)) & ~63u;
             first = first < kChunk ? kChunk : (first > 4096u ? 4096u : first);
@@ -681,6 +693,31 @@ __device__ __forceinline__ void set_open_count(LeafLds& L, int tid, uint32_t n) 
     __hip_atomic_store(&L.open.n[tid >> 6], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
+// Ends an occlusion ray: its flag, or (connecting) a place on the list if it
+// is not occluded.
+template <bool kConnect>
+__device__ __forceinline__ void finish_any(const TraceArgs& args, LeafLds& L, uint32_t ray, bool occl, int tid) {
+    if (!kConnect) {
+        args.occl[ray] = occl ? 1u : 0u;
+        return;
+    }
+    const unsigned long long m = __ballot(!occl);
+    if (!occl) {
+        const uint32_t base = open_count(L, tid);
+        L.open.ray[tid >> 6][base + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] = ray;
+        __builtin_amdgcn_wave_barrier();
+        set_open_count(L, tid, base + (uint32_t)__popcll(m));
+    }
+}
+
+// A split ray's slot, written by other lanes of the wave.
+__device__ __forceinline__ unsigned long long skey_load(unsigned long long* key, uint32_t i) {
+    return __hip_atomic_load(&key[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+__device__ __forceinline__ void skey_store(unsigned long long* key, uint32_t i, unsigned long long v) {
+    __hip_atomic_store(&key[i], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // Adds the contributions of up to 64 of the wave's listed unoccluded rays to
 // their paths (the last ones of the list) and shortens the list.  Every lane
 // of the wave must call it.
@@ -725,7 +762,7 @@ __device__ __forceinline__ void connect_open(const TraceArgs& args, LeafLds& L, 
 // before any of these switches, so a set is always tested in the space and
 // with the primitive base it was found in.
 //
-// Split rays (closest hit, one level): once the rays are handed out, lanes
+// Split rays (kSplit; one level): once the rays are handed out, lanes
 // whose rays are done would idle while the wave finishes its longest rays.
 // Such a lane takes the top group entry of a lane still at work and
 // traverses that group for the same ray (reloaded from the ray buffer) with
@@ -736,17 +773,23 @@ __device__ __forceinline__ void connect_open(const TraceArgs& args, LeafLds& L, 
 // writes the ray's hit once no helper of its ray is left.  The result is the
 // minimum key over all triangles the ray hits in [tmin, tmax], the same as
 // without splitting.  A helper also culls with its owner's closest distance
-// once that is nearer (read at every pass of the drain phase).  Occlusion
-// does not split: split occlusion rays made the integrator 2 % slower.
+// once that is nearer (read at every pass of the drain phase).  An occlusion
+// ray's slot holds only whether a part of it has hit; its helpers then stop.
+// Occlusion splits in the integrator's pair launches (with 96 registers they
+// have room for it; terrain render 15.70 -> 15.55 ms, guided room 6.11 -> 6.04)
+// and, in launches of its own, up to kSplitRays rays per block: 2,000 / 65,536
+// / 200,000 rays 75 / 92 / 125 us without, 71 / 77 / 92 with; at 1,000,003 rays
+// three launches in flight take 164 us each with and 150 without (the loop has
+// five spilled registers), at 400,000 84 and 80.
 //
 // Connect (kConnect, occlusion): instead of a flag per ray, a ray that is not
 // occluded adds its contribution to its path's radiance.  The finished rays
 // are listed in LDS and added 64 at a time, so the two dependent loads
 // (contribution, radiance) are waited for once per 64 rays, not once per
 // loop pass.  A path has at most one ray in the queue: no two adds meet.
-template <bool kAny, bool kCount, bool kInst, bool kConnect = false>
+template <bool kAny, bool kCount, bool kInst, bool kConnect = false, bool kSplit = !kAny && !kInst>
 __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uint32_t block, uint32_t blocks) {
-    constexpr bool kSplit = !kAny && !kInst;
+    static_assert(!(kSplit && kInst), "the split state and the world-space rays share their LDS");
     LeafLds& leafl = S.leaf;
     float4 (&wray)[2][KP_TRACE_BLOCK] = S.wray;
     unsigned long long (&skey)[KP_TRACE_BLOCK] = S.split.key;
@@ -778,7 +821,9 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
     bool split_on = false;   // rays are being split (wave-uniform; roles live in srole)
     uint64_t cnt_nodes = 0, cnt_tris = 0;
     RayFeeder feed;
-    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks);
+    // (the counted variant measures the visits a ray needs: no thin launches,
+    // which trade visits for latency, +28 % on 4,096 rays)
+    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kSplit && !kAny && !kCount);
     if (kConnect) {
         set_open_count(leafl, tid, 0u);
         __builtin_amdgcn_wave_barrier();
@@ -824,6 +869,17 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 skey[tid] = ~0ull;
             }
             uint32_t role = srole[tid];
+            if (kAny) {
+                // a part of the ray has hit: its helpers stop, its owner waits for that
+                const bool hit = ray_id != KP_INVALID && skey_load(skey, role & 0xFFu) != ~0ull;
+                if (hit && (role & kHelper)) {
+                    ray_id = KP_INVALID;
+                } else if (hit && !(role & kWaiting)) {
+                    role |= kWaiting;
+                    srole[tid] = role;
+                    steps = kStepsWaiting;
+                }
+            }
             unsigned long long* busy_w = &sbusy[tid >> 6];
             if (__ballot(ray_id != KP_INVALID && (role & kWaiting)) != 0ull) {
                 // owners whose helpers are all done write their ray's hit (the
@@ -835,12 +891,16 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 __builtin_amdgcn_wave_barrier();
                 const unsigned long long busy = __hip_atomic_load(busy_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
                 if (ray_id != KP_INVALID && (role & kWaiting) && !((busy >> lane) & 1ull)) {
-                    const unsigned long long k = skey[tid], own = leafl.key[tid];
-                    write_hit(args.hits + ray_id, k < own ? k : own, k < own ? shit[tid] : leafl.hit[tid]);
+                    if (kAny) {
+                        finish_any<kConnect>(args, leafl, ray_id, skey_load(skey, tid) != ~0ull, tid);
+                    } else {
+                        const unsigned long long k = skey[tid], own = leafl.key[tid];
+                        write_hit(args.hits + ray_id, k < own ? k : own, k < own ? shit[tid] : leafl.hit[tid]);
+                    }
                     ray_id = KP_INVALID;
                 }
             }
-            {
+            if (!kAny) {
                 // a helper culls with its owner's closest distance once that
                 // is nearer; its own hit, farther than the owner's, cannot win
                 const float ob = __shfl(best_t, (int)(role & 63u));
@@ -878,7 +938,8 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                         setup_ray(args.rays[2 * (size_t)rid], args.rays[2 * (size_t)rid + 1], r);
                         nt = node_test_setup(r);
                         best_t = bt;
-                        leafl.key[tid] = ~0ull;
+                        if (!kAny) leafl.key[tid] = ~0ull;
+                        occl = false;
                         pend = 0u;
                         cur = KP_INVALID;
                         steps = 0;
@@ -891,6 +952,8 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
         if (__ballot(ray_id != KP_INVALID || feed.pid != KP_INVALID) == 0) break;
         // an owner waiting for its helpers has steps == kStepsWaiting
         if (ray_id != KP_INVALID && steps != kStepsWaiting) {
+            // nothing left to hand out and nothing to split: run to the end
+            const bool more = !feed.drained || __ballot(feed.pid != KP_INVALID) != 0ull;
             for (;;) {
                 bool fault = false;
                 uint32_t pend2 = 0u;   // a second leaf set found this iteration
@@ -1027,17 +1090,18 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 }
                 if (done) {
                     const uint32_t role = kSplit && split_on ? srole[tid] : 0u;
-                    if (kConnect) {
-                        const unsigned long long m = __ballot(!occl);
-                        if (!occl) {
-                            const uint32_t base = open_count(leafl, tid);
-                            leafl.open.ray[tid >> 6][base + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] =
-                                ray_id;
-                            __builtin_amdgcn_wave_barrier();
-                            set_open_count(leafl, tid, base + (uint32_t)__popcll(m));
+                    if (kAny) {
+                        if (kSplit && (role & kHelper)) {
+                            if (occl) skey_store(skey, role & 0xFFu, 0ull);
+                        } else if (kSplit && (role & kDonated)) {
+                            if (occl) skey_store(skey, tid, 0ull);
+                            srole[tid] = role | kWaiting;   // finished once the helpers are done
+                            steps = kStepsWaiting;
+                            pend = 0u;
+                            break;
+                        } else {
+                            finish_any<kConnect>(args, leafl, ray_id, occl, tid);
                         }
-                    } else if (kAny) {
-                        args.occl[ray_id] = occl ? 1u : 0u;
                     } else if (kSplit && (role & kHelper)) {
                         // merge into the owner's slot: minimum key, then the
                         // t, u, v of the lane whose key is the minimum
@@ -1061,13 +1125,15 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                     pend = 0u;
                     break;
                 }
-                if (__popcll(__ballot(true)) < args.refill_below) break;
+                if (__popcll(__ballot(true)) < args.refill_below && (kSplit || more)) break;
             }
         }
     }
     if (kConnect) {
-        const uint32_t open = open_count(leafl, tid);
-        if (open != 0u) connect_open(args, leafl, open, tid);
+        // (waiting owners may have joined the list after the pass's check, so
+        // up to 127 rays are left)
+        for (uint32_t open = open_count(leafl, tid); open != 0u; open = open_count(leafl, tid))
+            connect_open(args, leafl, open, tid);
     }
     if (kCount) {
         atomicAdd((unsigned long long*)&args.counters[0], (unsigned long long)cnt_nodes);
@@ -1096,10 +1162,11 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
     traverse<false, false, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
+template <bool kSplit>
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_occluded5(
     TraceArgs args) {
     __shared__ TraceLds lds;
-    traverse<true, false, false>(args, lds, blockIdx.x, gridDim.x);
+    traverse<true, false, false, false, kSplit>(args, lds, blockIdx.x, gridDim.x);
 }
 
 // The two-level traversals compiled for 5 waves per SIMD (96 registers, 44 B
@@ -1140,7 +1207,7 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
         args.roots = q.roots;
         args.scontrib = q.contrib;
         args.radiance = q.radiance;
-        traverse<true, false, kInst, true>(args, lds, blockIdx.x - n_closest, gridDim.x - n_closest);
+        traverse<true, false, kInst, true, !kInst>(args, lds, blockIdx.x - n_closest, gridDim.x - n_closest);
     }
 }
 
@@ -1175,9 +1242,17 @@ __global__ void k_reset_u32(uint32_t* p, uint32_t n) {
 }
 
 // ---------------------------------------------------------------- launch --
+// Whether the launch's feeders take rays from the counter: not while first
+// chunks hold every ray (RayFeeder::init), so small launches need no clearing
+// launch before them (5 us; 1,000 rays with three launches in flight 11.3 us
+// a launch with it).
+static bool uses_counter(const TraceArgs& a, uint32_t grid) {
+    return a.n_dev || (uint64_t)a.n > (uint64_t)grid * (KP_TRACE_BLOCK / 64) * kChunk;
+}
+
 hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool reset, hipStream_t s) {
     if (grid == 0 || grid > a.spill_blocks) return hipErrorInvalidValue;   // lanes without a spill slice
-    if (reset) hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
+    if (reset && uses_counter(a, grid)) hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
     if (a.insts) {
         if (count) hipLaunchKernelGGL(k_closest_inst<true>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
         else if (a.five_waves) hipLaunchKernelGGL(k_closest_inst5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
@@ -1192,10 +1267,12 @@ hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool re
 
 hipError_t launch_occluded(const TraceArgs& a, uint32_t grid, hipStream_t s) {
     if (grid == 0 || grid > a.spill_blocks) return hipErrorInvalidValue;   // lanes without a spill slice
-    hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
+    if (uses_counter(a, grid)) hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
     if (a.insts && a.five_waves) hipLaunchKernelGGL(k_occluded_inst5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
     else if (a.insts) hipLaunchKernelGGL(k_occluded_inst, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
-    else if (a.five_waves) hipLaunchKernelGGL(k_occluded5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
+    else if (a.five_waves && !a.n_dev && (uint64_t)a.n <= (uint64_t)grid * kSplitRays)
+        hipLaunchKernelGGL(k_occluded5<true>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
+    else if (a.five_waves) hipLaunchKernelGGL(k_occluded5<false>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
     else hipLaunchKernelGGL(k_occluded, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
     return hipGetLastError();
 }
@@ -1226,7 +1303,7 @@ hipError_t trace_occupancy_five(int* blocks_per_cu_closest, int* blocks_per_cu_o
     if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&two, k_closest_inst5, KP_TRACE_BLOCK, 0);
     if (e != hipSuccess) return e;
     *blocks_per_cu_closest = one < two ? one : two;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&one, k_occluded5, KP_TRACE_BLOCK, 0);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&one, k_occluded5<true>, KP_TRACE_BLOCK, 0);
     if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&two, k_occluded_inst5, KP_TRACE_BLOCK, 0);
     if (e != hipSuccess) return e;
     *blocks_per_cu_occluded = one < two ? one : two;

@@ -50,3 +50,42 @@ def test_path_counts_around_the_edges(two_level, depth):
     # a repeat gives the same bits
     assert np.array_equal(c.integrate_rays(rays, d).view(np.uint32), big.view(np.uint32))
     c.close()
+
+
+COUNTS = (1, 3, 4, 5, 63, 64, 65, 1025, 4099, 65535, 65537, 327679, 327681)
+
+
+def test_small_launches_split_their_rays():
+    """Launches of one wave per SIMD and fewer, with rays split among lanes
+    (closest hit and occlusion), at counts around each rule's limits: the host
+    traversal of the same BVH gives the same bits."""
+    rng = np.random.default_rng(21)
+    c = native.Context(0)
+    c.mesh_add_soup(scenes.microbench_triangles(seed=4, n_lon=64, n_lat=32, n_random=6000))
+    c.bvh_build()
+    rays = scenes.incoherent_rays(max(COUNTS), rng)
+    rays[::3, 7] = rng.uniform(0.05, 1.0, rays[::3].shape[0])
+    rays[5::11, 3] = -0.2
+    hits, occ = c.intersect_closest_host(rays), c.occluded_host(rays)
+    assert 0.2 < occ.mean() < 0.9
+    for n in COUNTS:
+        assert np.array_equal(c.intersect_closest(rays[:n]).view(np.uint32), hits[:n].view(np.uint32)), n
+        assert np.array_equal(c.occluded(rays[:n]), occ[:n]), n
+    c.close()
+
+
+def test_split_occlusion_with_spilled_stacks():
+    """A tree whose pending groups exceed the LDS stack: groups are handed to
+    idle lanes from stacks that have spilled to memory."""
+    from test_deep_bvh import deep_rays, deep_scene
+    t = deep_scene()
+    rays = deep_rays(3000)
+    rays[1::4, 7] = 1.5
+    c = native.Context(0)
+    c.mesh_add_soup(t)
+    c.bvh_build()
+    for n in (64, 127, 2000, rays.shape[0]):
+        assert np.array_equal(c.occluded(rays[:n]), c.occluded_host(rays[:n])), n
+        assert np.array_equal(c.intersect_closest(rays[:n]).view(np.uint32),
+                              c.intersect_closest_host(rays[:n]).view(np.uint32)), n
+    c.close()

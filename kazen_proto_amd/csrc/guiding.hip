@@ -187,111 +187,149 @@ __host__ __device__ constexpr int g_tile_base(int l) {
 #define KP_G_TILES 68
 #define KP_G_WTILES 17
 
-// Eight consecutive samples s0 .. s0 + 7 of column f of a sample-major bf16
-// block (row stride KP_G_ROW words), packed two per word in sample order: the
-// matrix-core operand with samples along k, gathered by 16-bit LDS reads.
-__device__ __forceinline__ u32x4 g_column8(const uint32_t* rows, int s0, int f) {
-    const uint16_t* p = reinterpret_cast<const uint16_t*>(rows + s0 * KP_G_ROW) + f;
-    constexpr int st = 2 * KP_G_ROW;   // row stride in halves
-    u32x4 v;
-    v[0] = (uint32_t)p[0] | ((uint32_t)p[st] << 16);
-    v[1] = (uint32_t)p[2 * st] | ((uint32_t)p[3 * st] << 16);
-    v[2] = (uint32_t)p[4 * st] | ((uint32_t)p[5 * st] << 16);
-    v[3] = (uint32_t)p[6 * st] | ((uint32_t)p[7 * st] << 16);
-    return v;
+// Samples s0 .. s0 + 7 (s0 = 8 g + a multiple of 32 for lane group g) of the 16
+// columns f0 .. f0 + 15 of a sample-major bf16 block (row stride KP_G_ROW
+// words): lane r of the group receives column f0 + r, two samples per word in
+// sample order, the matrix-core operand with samples along k.  Two transposing
+// LDS reads (a group's 16 lanes name four rows of 16 values, four consecutive
+// values each, and receive one column each).
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 g_column8(const uint32_t* rows, int s0, int f0, int r) {
+    typedef __attribute__((address_space(3))) i16x4 lds4;
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(rows + (s0 + (r >> 2)) * KP_G_ROW) + f0 + 4 * (r & 3);
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p);
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(p + 8 * KP_G_ROW));   // four rows on
+    const uint2 l = __builtin_bit_cast(uint2, lo), h = __builtin_bit_cast(uint2, hi);
+    return u32x4{l.x, l.y, h.x, h.y};
 }
 
-// dW[k][n] += sum over the group's 64 samples of X[s][k] dY[s][n]: A = X^T
-// (16 features x 32 samples), B = dY (32 samples x 16 outputs), both gathered
-// from the sample-major blocks (no transposed copies: they would double the
-// block's LDS and keep it at one block per CU).
-template <int L>
-__device__ __forceinline__ void g_dw_tiles(const uint32_t* X, const uint32_t* dY, int wave, int lane,
-                                           f32x4* acc) {
-    constexpr int ntn = g_dim_out(L) / 16;
-    const int g = lane >> 4, r = lane & 15;
+// The weight fragments one wave of a training block uses: forward n-tile
+// `wave` of layers 0-3 and `wave & 1` of layer 4, backward k-tile `wave`.
+struct TrainFrags {
+    u32x4 f[KP_G_LAYERS][2];
+    u32x4 b[KP_G_LAYERS][2];   // layers 1-4 (layer 4 has one)
+};
+
+__device__ __forceinline__ void g_load_frags(const GuideNet& net, int wave, int lane, TrainFrags& w) {
 #pragma unroll
-    for (int kt = 0; kt < g_ktiles(L); ++kt)
+    for (int l = 0; l < KP_G_LAYERS; ++l) {
+        const int nt = l < KP_G_LAYERS - 1 ? wave : wave & 1;
 #pragma unroll
-        for (int nt = 0; nt < ntn; ++nt) {
-            const int id = g_tile_base(L) + kt * ntn + nt;
-            if ((id & 3) != wave) continue;
-            f32x4 a = acc[id >> 2];
+        for (int c = 0; c < 2; ++c) w.f[l][c] = net.wf[(g_wf_base(l) + 2 * nt + c) * 64 + lane];
+        if (l > 0) {
+            const int nch = g_dim_out(l) / 32;
 #pragma unroll
-            for (int sc = 0; sc < 2; ++sc) {
-                const u32x4 av = g_column8(X, 32 * sc + 8 * g, 16 * kt + r);
-                const u32x4 bv = g_column8(dY, 32 * sc + 8 * g, 16 * nt + r);
-                a = mfma16(av, bv, a);
-            }
-            acc[id >> 2] = a;
+            for (int c = 0; c < nch; ++c) w.b[l][c] = net.wb[(g_wb_base(l) + wave * nch + c) * 64 + lane];
         }
+    }
 }
 
+// The four biases of layer L that lane group g adds in n-tile nt (read per
+// group, from the L1: the registers are taken).
 template <int L>
-__device__ __forceinline__ void g_dw_store(float* part, int wave, int lane, const f32x4* acc) {
-    constexpr int ntn = g_dim_out(L) / 16, dout = g_dim_out(L);
+__device__ __forceinline__ float4 g_bias(const float* params, int nt, int g) {
+    asm volatile("" : "+s"(params));   // not hoisted out of the group loop
+    return *reinterpret_cast<const float4*>(params + g_layer_offset(L) + g_dim_in(L) * g_dim_out(L) + 16 * nt + 4 * g);
+}
+
+// Outputs of one n-tile of layer L for the 16 samples of chunk c.
+template <int L>
+__device__ __forceinline__ f32x4 g_forward_tile(const uint32_t* x, const TrainFrags& w, const float4& bias, int c, int g,
+                                                int r) {
+    const uint32_t* row = x + (16 * c + r) * KP_G_ROW;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    acc = mfma16(w.f[L][0], *(const u32x4*)(row + 4 * g), acc);
+    acc = mfma16(w.f[L][1], *(const u32x4*)(row + 16 + 4 * g), acc);
+    acc[0] += bias.x;
+    acc[1] += bias.y;
+    acc[2] += bias.z;
+    acc[3] += bias.w;
+    return acc;
+}
+
+// One wave's part of hidden layer L: its n-tile for all 64 samples.
+template <int L>
+__device__ __forceinline__ void g_forward_layer(const float* params, const uint32_t* x, uint32_t* y,
+                                                const TrainFrags& w, int wave, int g, int r) {
+    const float4 bias = g_bias<L>(params, wave, g);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const f32x4 v = g_forward_tile<L>(x, w, bias, c, g, r);
+        *reinterpret_cast<uint2*>(y + (16 * c + r) * KP_G_ROW + 8 * wave + 2 * g) =
+            make_uint2(pack_bf2(fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f)), pack_bf2(fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)));
+    }
+}
+
+// Back-propagation through layer L for one 64-sample group.  The wave's share
+// is its n-tile of the weight gradient, dW[k][n] += sum over the samples of
+// X[s][k] dY[s][n] (A = X^T, 16 features x 32 samples, B = dY; layer 4 has two
+// n-tiles, so its waves share the k-tiles), the same tile's bias gradient
+// (A = ones), and, for L > 0, k-tile `wave` of dX = (W dY) masked by the ReLU of
+// the layer input, for all 64 samples.
+template <int L>
+__device__ __forceinline__ void g_backward_layer(const TrainFrags& w, const uint32_t* X, const uint32_t* dY, uint32_t* dX,
+                                                 int wave, int lane, f32x4* acc, f32x4* bacc) {
     const int g = lane >> 4, r = lane & 15;
-    float* gW = part + g_layer_offset(L);
+    constexpr bool last = L == KP_G_LAYERS - 1;
+    const int nt = last ? wave & 1 : wave;
+    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
 #pragma unroll
-    for (int kt = 0; kt < g_ktiles(L); ++kt)
+    for (int sc = 0; sc < 2; ++sc) {
+        const u32x4 bv = g_column8(dY, 32 * sc + 8 * g, 16 * nt, r);
+        bacc[L] = mfma16(ones, bv, bacc[L]);
 #pragma unroll
-        for (int nt = 0; nt < ntn; ++nt) {
-            const int id = g_tile_base(L) + kt * ntn + nt;
-            if ((id & 3) != wave) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) gW[(16 * kt + 4 * g + j) * dout + 16 * nt + r] = acc[id >> 2][j];
+        for (int i = 0; i < (last ? 2 : g_ktiles(L)); ++i) {
+            const int kt = last ? (wave >> 1) + 2 * i : i;
+            f32x4& a = acc[g_tile_base(L) / 4 + i];
+            a = mfma16(g_column8(X, 32 * sc + 8 * g, 16 * kt, r), bv, a);
         }
-}
-
-// Back-propagation through layer L for one 64-sample group: accumulate its
-// weight and bias gradients, then (L > 0) write dX = (W dY) masked by the
-// ReLU of the layer input, sample-major, for this wave's 16 samples.
-template <int L>
-__device__ __forceinline__ void g_backward_layer(const GuideNet& net, uint32_t (*act)[64 * KP_G_ROW],
-                                                 const uint32_t* dY, uint32_t* dX, int tid, int wave, int lane,
-                                                 f32x4* acc, float* bacc) {
-    constexpr int dout = g_dim_out(L);
-    g_dw_tiles<L>(act[L], dY, wave, lane, acc);
-    if (tid < dout) {
-        // bias gradient: column tid of dY, summed in sample order
-        float sb = bacc[L];
-        const uint16_t* col = reinterpret_cast<const uint16_t*>(dY) + tid;
-#pragma unroll 8
-        for (int s = 0; s < 64; ++s) sb += __uint_as_float((uint32_t)col[s * 2 * KP_G_ROW] << 16);
-        bacc[L] = sb;
     }
     if constexpr (L > 0) {
-        const int g = lane >> 4, r = lane & 15;
-        constexpr int nch = dout / 32;
-        const uint32_t* dyrow = dY + (16 * wave + r) * KP_G_ROW;
-        const uint32_t* xrow = act[L] + (16 * wave + r) * KP_G_ROW;
-        uint32_t* dxrow = dX + (16 * wave + r) * KP_G_ROW;
+        constexpr int nch = g_dim_out(L) / 32;
+        const int k0 = 16 * wave + 4 * g;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
+        for (int c = 0; c < 4; ++c) {
+            const int row = (16 * c + r) * KP_G_ROW;
             f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int c = 0; c < nch; ++c) {
-                const u32x4 b = *(const u32x4*)(dyrow + 16 * c + 4 * g);
-                d = mfma16(net.wb[(g_wb_base(L) + kt * nch + c) * 64 + lane], b, d);
-            }
-            const int k0 = 16 * kt + 4 * g;
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t xw = xrow[(k0 + j) >> 1];
-                const float xv = ((k0 + j) & 1) ? bf_hi(xw) : bf_lo(xw);
-                v[j] = xv > 0.0f ? d[j] : 0.0f;
-            }
-            dxrow[k0 / 2] = pack_bf2(v[0], v[1]);
-            dxrow[k0 / 2 + 1] = pack_bf2(v[2], v[3]);
+            for (int h = 0; h < nch; ++h) d = mfma16(w.b[L][h], *(const u32x4*)(dY + row + 16 * h + 4 * g), d);
+            const uint2 xw = *reinterpret_cast<const uint2*>(X + row + k0 / 2);
+            const float v0 = bf_lo(xw.x) > 0.0f ? d[0] : 0.0f, v1 = bf_hi(xw.x) > 0.0f ? d[1] : 0.0f;
+            const float v2 = bf_lo(xw.y) > 0.0f ? d[2] : 0.0f, v3 = bf_hi(xw.y) > 0.0f ? d[3] : 0.0f;
+            *reinterpret_cast<uint2*>(dX + row + k0 / 2) = make_uint2(pack_bf2(v0, v1), pack_bf2(v2, v3));
         }
     }
+}
+
+// Writes the wave's tiles of layer L into the block's partial gradient.
+template <int L>
+__device__ __forceinline__ void g_grad_store(float* part, int wave, int lane, const f32x4* acc, const f32x4* bacc) {
+    constexpr int dout = g_dim_out(L);
+    constexpr bool last = L == KP_G_LAYERS - 1;
+    const int g = lane >> 4, r = lane & 15, nt = last ? wave & 1 : wave;
+    float* gW = part + g_layer_offset(L);
+#pragma unroll
+    for (int i = 0; i < (last ? 2 : g_ktiles(L)); ++i) {
+        const int kt = last ? (wave >> 1) + 2 * i : i;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) gW[(16 * kt + 4 * g + j) * dout + 16 * nt + r] = acc[g_tile_base(L) / 4 + i][j];
+    }
+    if (g == 0 && (!last || wave < 2)) gW[g_dim_in(L) * dout + 16 * nt + r] = bacc[L][0];
 }
 
 // Persistent training blocks: block b runs the 64-sample groups b, b + grid,
-// ... (4 waves x 16 samples each), keeps its weight-gradient tiles in the
-// matrix-core accumulators and its bias gradients in registers across groups,
-// and writes one partial gradient (canonical layout) to partial[b].
+// ..., keeps its weight- and bias-gradient tiles in the matrix-core
+// accumulators across groups, and writes one partial gradient (canonical
+// layout) to partial[b].
+//
+// A layer's output tiles are split over the block's four waves (not its
+// samples), so a wave uses the same 17 weight fragments for every group and
+// keeps them in registers; with the samples split, every wave read all 64
+// fragments (64 KB) for every 16 samples.  Operands with samples along k come
+// from transposing LDS reads instead of eight 16-bit reads each.  At 262,144
+// samples: 197 us before, 119 now (27.4 GFLOP of algorithmic work, 230 TFLOP/s); what
+// is left is the chain of about 14 barriers a group and the output gradient's
+// transcendentals at two waves per SIMD.
 __global__ __launch_bounds__(256, 2) void k_guide_train(GuideNet net, const float* __restrict__ in6,
                                                         const float* __restrict__ dirs,
                                                         const float* __restrict__ weights,
@@ -305,12 +343,15 @@ __global__ __launch_bounds__(256, 2) void k_guide_train(GuideNet net, const floa
     float* outs = reinterpret_cast<float*>(dyb[1]);
     const uint32_t n = *n_dev;
     const uint32_t groups = (n + 63) / 64;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = __lane_id();
+    const int tid = threadIdx.x, wave = tid >> 6, lane = __lane_id(), g = lane >> 4, r = lane & 15;
     const float scale = *scale_dev;
-    f32x4 acc[KP_G_WTILES];
+    TrainFrags w;
+    g_load_frags(net, wave, lane, w);
+    f32x4 acc[KP_G_WTILES], bacc[KP_G_LAYERS];
 #pragma unroll
     for (int i = 0; i < KP_G_WTILES; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bacc[KP_G_LAYERS] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < KP_G_LAYERS; ++i) bacc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     for (uint32_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
         const uint32_t base = grp * 64;
@@ -343,10 +384,21 @@ __global__ __launch_bounds__(256, 2) void k_guide_train(GuideNet net, const floa
             row[25 + 2 * part] = 0u;
         }
         __syncthreads();
-        {
-            uint32_t* a[4] = {act[1] + 16 * wave * KP_G_ROW, act[2] + 16 * wave * KP_G_ROW,
-                              act[3] + 16 * wave * KP_G_ROW, act[4] + 16 * wave * KP_G_ROW};
-            g_forward_chunk(net, act[0] + 16 * wave * KP_G_ROW, a, outs + 16 * wave * KP_G_ROW, KP_G_ROW);
+        g_forward_layer<0>(net.params, act[0], act[1], w, wave, g, r);
+        __syncthreads();
+        g_forward_layer<1>(net.params, act[1], act[2], w, wave, g, r);
+        __syncthreads();
+        g_forward_layer<2>(net.params, act[2], act[3], w, wave, g, r);
+        __syncthreads();
+        g_forward_layer<3>(net.params, act[3], act[4], w, wave, g, r);
+        __syncthreads();
+        const float4 bias4 = g_bias<4>(net.params, wave & 1, g);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {   // two n-tiles: each wave takes one of them for half the samples
+            const int c = 2 * (wave >> 1) + i;
+            const f32x4 v = g_forward_tile<4>(act[4], w, bias4, c, g, r);
+            *reinterpret_cast<float4*>(outs + (16 * c + r) * KP_G_ROW + 16 * (wave & 1) + 4 * g) =
+                make_float4(v[0], v[1], v[2], v[3]);
         }
         __syncthreads();
         {
@@ -369,26 +421,23 @@ __global__ __launch_bounds__(256, 2) void k_guide_train(GuideNet net, const floa
             for (int w = 16 + 4 * part; w < 20 + 4 * part; ++w) row[w] = 0u;
         }
         __syncthreads();
-        g_backward_layer<4>(net, act, dyb[0], dyb[1], tid, wave, lane, acc, bacc);
+        g_backward_layer<4>(w, act[4], dyb[0], dyb[1], wave, lane, acc, bacc);
         __syncthreads();
-        g_backward_layer<3>(net, act, dyb[1], dyb[0], tid, wave, lane, acc, bacc);
+        g_backward_layer<3>(w, act[3], dyb[1], dyb[0], wave, lane, acc, bacc);
         __syncthreads();
-        g_backward_layer<2>(net, act, dyb[0], dyb[1], tid, wave, lane, acc, bacc);
+        g_backward_layer<2>(w, act[2], dyb[0], dyb[1], wave, lane, acc, bacc);
         __syncthreads();
-        g_backward_layer<1>(net, act, dyb[1], dyb[0], tid, wave, lane, acc, bacc);
+        g_backward_layer<1>(w, act[1], dyb[1], dyb[0], wave, lane, acc, bacc);
         __syncthreads();
-        g_backward_layer<0>(net, act, dyb[0], nullptr, tid, wave, lane, acc, bacc);
+        g_backward_layer<0>(w, act[0], dyb[0], nullptr, wave, lane, acc, bacc);
         __syncthreads();
     }
     float* part = partial + (size_t)blockIdx.x * KP_G_PARAMS;
-    g_dw_store<0>(part, wave, lane, acc);
-    g_dw_store<1>(part, wave, lane, acc);
-    g_dw_store<2>(part, wave, lane, acc);
-    g_dw_store<3>(part, wave, lane, acc);
-    g_dw_store<4>(part, wave, lane, acc);
-#pragma unroll
-    for (int l = 0; l < KP_G_LAYERS; ++l)
-        if (tid < g_dim_out(l)) part[g_layer_offset(l) + g_dim_in(l) * g_dim_out(l) + tid] = bacc[l];
+    g_grad_store<0>(part, wave, lane, acc, bacc);
+    g_grad_store<1>(part, wave, lane, acc, bacc);
+    g_grad_store<2>(part, wave, lane, acc, bacc);
+    g_grad_store<3>(part, wave, lane, acc, bacc);
+    g_grad_store<4>(part, wave, lane, acc, bacc);
 }
 
 // First stage of the gradient reduction: seg[s][p] = sum over partials

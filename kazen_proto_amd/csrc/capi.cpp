@@ -53,7 +53,7 @@ TraceArgs trace_base(kp_ctx* c) {
     a.counter = c->d_words;
     a.err = c->d_words + 1;
     a.spill = c->d_spill;
-    a.spill_cap = c->spill_cap;
+    a.spill_cap = c->spill_area;
     a.spill_blocks = (uint32_t)(c->spill_lanes / KP_TRACE_BLOCK);
     a.refill_below = c->refill_below;
     a.counters = c->d_counters;
@@ -65,6 +65,22 @@ TraceArgs trace_base(kp_ctx* c) {
         a.world_root = c->world_root;
     }
     return a;
+}
+
+int finish(kp_ctx* c, const unsigned long long* totals, const uint32_t* train_records) {
+    uint32_t* noalloc_err = c->noalloc_used ? (uint32_t*)(c->d_scratch + KP_SCRATCH_ERR_OFFSET) : nullptr;
+    KP_HIP_TRY(c, launch_status(c->d_words + 1, noalloc_err, totals, train_records, c->h_status, c->stream));
+    KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
+    const uint32_t flags = c->h_status->err | c->h_status->noalloc_err;
+    if (flags) {
+        if (c->h_status->noalloc_err) KP_HIP_TRY(c, launch_reset_u32(noalloc_err, 1u, c->stream));
+        KP_HIP_TRY(c, launch_reset_u32(c->d_words + 1, 1u, c->stream));
+        KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
+        return fail(c, KP_ERR_KERNEL,
+                    (flags & 1u) ? "traversal stack exceeded its spill capacity"
+                                 : "traversal exceeded its step limit");
+    }
+    return KP_OK;
 }
 
 int trace_closest_dev(kp_ctx* c, const float4* rays, uint32_t n, float4* hits, bool count) {
@@ -300,6 +316,7 @@ static int build_two_level(kp_ctx* c, const BuildOptions& bo, double* seconds) {
     // return marker, 7 per prototype level.
     // Postponed leaves need no stack entries.
     c->spill_cap = 8u * top.max_depth + 7u * max_unit_depth + 16u;
+    c->spill_area = 8u * top.max_depth + max_unit_depth + 16u;   // one group per prototype level
     if (c->device >= 0) {
         const size_t tbytes = tris.size() * sizeof(float);
         const int urc = upload_nodes(c, nodes);
@@ -312,7 +329,7 @@ static int build_two_level(kp_ctx* c, const BuildOptions& bo, double* seconds) {
         KP_HIP_TRY(c, hipMemcpy(c->d_tlas_inst, top.tri_order.data(), top.tri_order.size() * 4,
                                 hipMemcpyHostToDevice));
         c->spill_lanes = (size_t)kp::max_trace_grid(c) * KP_TRACE_BLOCK;
-        KP_HIP_TRY(c, hipMalloc((void**)&c->d_spill, c->spill_lanes * c->spill_cap * sizeof(uint2)));
+        KP_HIP_TRY(c, hipMalloc((void**)&c->d_spill, c->spill_lanes * c->spill_area * sizeof(uint2)));
     }
     c->two_level = true;
     c->world_root = has_world ? node_off[0] : KP_INVALID;
@@ -375,6 +392,8 @@ int kp_create(kp_ctx** out, int device) {
     if ((e = hipMalloc((void**)&c->d_words, 64)) != hipSuccess) return bail(e, "alloc");
     if ((e = hipMemsetAsync(c->d_words, 0, 64, c->stream)) != hipSuccess) return bail(e, "memset");
     if ((e = hipMalloc((void**)&c->d_counters, 64)) != hipSuccess) return bail(e, "alloc");
+    if ((e = hipHostMalloc((void**)&c->h_status, sizeof(kp::HostStatus), hipHostMallocDefault)) != hipSuccess)
+        return bail(e, "alloc");
     if ((e = hipMemsetAsync(c->d_counters, 0, 64, c->stream)) != hipSuccess) return bail(e, "memset");
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return bail(e, "memset");
     int bc = 0, bo = 0;
@@ -412,6 +431,7 @@ void kp_destroy(kp_ctx* c) {
     kp::free_bvh(c);
     if (c->d_words) (void)hipFree(c->d_words);
     if (c->d_counters) (void)hipFree(c->d_counters);
+    if (c->h_status) (void)hipHostFree(c->h_status);
     if (c->d_stage_in) (void)hipFree(c->d_stage_in);
     if (c->d_stage_out) (void)hipFree(c->d_stage_out);
     if (c->ev_begin) (void)hipEventDestroy(c->ev_begin);
@@ -433,24 +453,7 @@ int kp_set_stream(kp_ctx* c, void* s) {
 int kp_synchronize(kp_ctx* c) {
     if (!c) return KP_ERR_INVALID;
     KP_USE_DEVICE(c);
-    KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
-    uint32_t flags = 0;
-    KP_HIP_TRY(c, hipMemcpy(&flags, c->d_words + 1, 4, hipMemcpyDeviceToHost));
-    if (c->noalloc_used) {   // errors of kp_intersect_closest_noalloc launches
-        uint32_t f2 = 0;
-        uint32_t* ew = (uint32_t*)(c->d_scratch + KP_SCRATCH_ERR_OFFSET);
-        KP_HIP_TRY(c, hipMemcpy(&f2, ew, 4, hipMemcpyDeviceToHost));
-        if (f2) KP_HIP_TRY(c, kp::launch_reset_u32(ew, 1u, c->stream));
-        flags |= f2;
-    }
-    if (flags) {
-        KP_HIP_TRY(c, hipMemsetAsync(c->d_words + 1, 0, 4, c->stream));
-        KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
-        return kp::fail(c, KP_ERR_KERNEL,
-                        (flags & 1u) ? "traversal stack exceeded its spill capacity"
-                                     : "traversal exceeded its step limit");
-    }
-    return KP_OK;
+    return kp::finish(c, nullptr, nullptr);
 }
 
 int kp_mesh_add(kp_ctx* c, const float* xyz, uint32_t n_verts, const uint32_t* idx,
@@ -659,6 +662,7 @@ static int install_one_level(kp_ctx* c, kp::Bvh8Host& h, uint32_t n_all, uint32_
     // Worst-case stack: 7 pushes per level below the root, plus slack; the
     // top KP_TRACE_STACK entries live in LDS.
     c->spill_cap = 7u * h.max_depth + 8u;
+    c->spill_area = kp::one_level_spill(h.max_depth);
     if (c->device >= 0) {
         const size_t tb = h.tris.size() * sizeof(float);
         const int urc = kp::upload_nodes(c, h.nodes);
@@ -666,7 +670,7 @@ static int install_one_level(kp_ctx* c, kp::Bvh8Host& h, uint32_t n_all, uint32_
         KP_HIP_TRY(c, hipMalloc((void**)&c->d_tris, tb));
         KP_HIP_TRY(c, hipMemcpy(c->d_tris, h.tris.data(), tb, hipMemcpyHostToDevice));
         c->spill_lanes = (size_t)kp::max_trace_grid(c) * KP_TRACE_BLOCK;
-        KP_HIP_TRY(c, hipMalloc((void**)&c->d_spill, c->spill_lanes * c->spill_cap * sizeof(uint2)));
+        KP_HIP_TRY(c, hipMalloc((void**)&c->d_spill, c->spill_lanes * c->spill_area * sizeof(uint2)));
     }
     c->n_tris_built = n_all;
     c->n_tris_stored = n_all;
@@ -919,6 +923,7 @@ int kp_intersect_closest_noalloc(kp_ctx* c, const kp_ray* rays, uint32_t n, kp_h
     a.rays = (const float4*)rays;
     a.hits = (float4*)hits;
     a.n = n;
+    a.spill_cap = c->spill_cap;
     a.counter = (uint32_t*)c->d_scratch;
     a.err = (uint32_t*)(c->d_scratch + KP_SCRATCH_ERR_OFFSET);
     a.spill = (uint2*)(c->d_scratch + KP_SCRATCH_SPILL_OFFSET);

@@ -55,7 +55,8 @@ struct kp_ctx {
     uint4* d_nodes = nullptr;
     float4* d_tris = nullptr;
     uint2* d_spill = nullptr;
-    uint32_t spill_cap = 0;
+    uint32_t spill_cap = 0;      // entries per lane: reported, and laid out in the static scratch
+    uint32_t spill_area = 0;     // entries per lane of d_spill
     size_t spill_lanes = 0;
     uint32_t grid_closest = 0, grid_occluded = 0;
     uint32_t shade_blocks = 0, shade_blocks_guided = 0;   // resident blocks of k_shade, whole device
@@ -66,6 +67,7 @@ struct kp_ctx {
 
     // small device words: [0] work counter, [1] error flags
     uint32_t* d_words = nullptr;
+    kp::HostStatus* h_status = nullptr;   // page-locked; written by the status kernel
     // this device's static scratch (kp_intersect_closest_noalloc), looked up at kp_create
     unsigned char* d_scratch = nullptr;
     bool noalloc_used = false;       // kp_synchronize also reads the scratch's error word
@@ -96,9 +98,17 @@ int ensure_buffer(kp_ctx* c, void** buf, size_t* cap, size_t bytes);
 // Trace helpers shared with the integrator (device pointers, async).
 int trace_closest_dev(kp_ctx* c, const float4* rays, uint32_t n, float4* hits, bool count);
 int trace_occluded_dev(kp_ctx* c, const float4* rays, uint32_t n, uint32_t* out);
+// Waits for the context's stream and reports kernel-detected errors; the
+// words given (device memory, may be NULL) are in c->h_status afterwards.
+int finish(kp_ctx* c, const unsigned long long* totals, const uint32_t* train_records);
 // Traversal arguments of the context's BVH (one- or two-level).
 TraceArgs trace_base(kp_ctx* c);
 uint32_t max_trace_grid(const kp_ctx* c);
+// Entries per lane that a one-level traversal of a tree of `depth` levels can
+// spill: a visit pushes at most one group and a level has at most one group
+// pending, so the stack never holds more than depth entries, the first
+// KP_TRACE_STACK of them in LDS (kept simple: those are not subtracted).
+inline uint32_t one_level_spill(uint32_t depth) { return depth + 2u; }
 // World-space triangles (9 floats each) of every primitive id: the
 // kp_mesh_add meshes, then each instance's prototype under its
 // object-to-world matrix, each coordinate ((m0 x + m1 y) + m2 z) + m3 in FP64

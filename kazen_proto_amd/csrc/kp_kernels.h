@@ -71,6 +71,18 @@ hipError_t launch_occluded(const TraceArgs& a, uint32_t grid, hipStream_t s);
 hipError_t trace_occupancy(int* blocks_per_cu_closest, int* blocks_per_cu_occluded);
 hipError_t trace_occupancy_five(int* blocks_per_cu_closest, int* blocks_per_cu_occluded);
 hipError_t shade_occupancy(int* blocks_per_cu_plain, int* blocks_per_cu_guided);
+// What the host reads after waiting for the stream (page-locked memory the
+// status kernel writes).
+struct HostStatus {
+    unsigned long long totals[2];   // integrator: extension and shadow rays
+    uint32_t err;                   // traversal error flags
+    uint32_t noalloc_err;           // the same of the static scratch
+    uint32_t train_records;
+    uint32_t pad;
+};
+// Copies the words that are not NULL into *out (0 for the others).
+hipError_t launch_status(const uint32_t* err, const uint32_t* noalloc_err, const unsigned long long* totals,
+                         const uint32_t* train_records, HostStatus* out, hipStream_t s);
 hipError_t launch_reset_u32(uint32_t* p, uint32_t n, hipStream_t s);
 // Device address of the static scratch on `device` (made current by the
 // caller), looked up once per device.

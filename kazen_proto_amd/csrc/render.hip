@@ -1310,10 +1310,9 @@ static int integrate_rays(kp_ctx* c, const kp_ray* rays, uint32_t n, const kp_re
             KP_HIP_TRY(c, hipMemcpyAsync(out + 3 * (size_t)off, d_out, (size_t)cnt * 12,
                                          hipMemcpyDeviceToHost, c->stream));
     }
-    if ((rc = kp_synchronize(c))) return rc;
+    if ((rc = finish(c, r->ps.totals, nullptr))) return rc;
     auto t1 = std::chrono::steady_clock::now();
-    unsigned long long tot[2];
-    KP_HIP_TRY(c, hipMemcpy(tot, r->ps.totals, 16, hipMemcpyDeviceToHost));
+    const unsigned long long* tot = c->h_status->totals;
     r->stats.paths = n;
     r->stats.extension_rays = tot[0];
     r->stats.shadow_rays = tot[1];
@@ -1423,10 +1422,9 @@ static int render_accumulate(kp_ctx* c, const kp_render_desc* d) {
         }
     }
     r->film_count += d->spp;
-    if ((rc = kp_synchronize(c))) return rc;
+    if ((rc = finish(c, r->ps.totals, steps ? g->rec_valid : nullptr))) return rc;
     auto t1 = std::chrono::steady_clock::now();
-    unsigned long long tot[2];
-    KP_HIP_TRY(c, hipMemcpy(tot, r->ps.totals, 16, hipMemcpyDeviceToHost));
+    const unsigned long long* tot = c->h_status->totals;
     r->stats.paths = (uint64_t)npix * d->spp;
     r->stats.extension_rays = tot[0];
     r->stats.shadow_rays = tot[1];
@@ -1435,8 +1433,7 @@ static int render_accumulate(kp_ctx* c, const kp_render_desc* d) {
     r->stats.paths_per_pass = n_paths;
     r->stats.train_steps = steps;
     r->stats.guided_passes = guided_passes;
-    r->stats.train_records = 0;
-    if (steps) KP_HIP_TRY(c, hipMemcpy(&r->stats.train_records, g->rec_valid, 4, hipMemcpyDeviceToHost));
+    r->stats.train_records = c->h_status->train_records;
     return KP_OK;
 }
 
@@ -1622,7 +1619,7 @@ static int batch_create(kp_ctx* c, kp_ctx* const* scenes, uint32_t n, BatchState
     b->n_nodes = on;
     b->n_tris = ot;
     b->bvh_depth = depth;
-    b->spill_cap = 7u * depth + 8u;
+    b->spill_cap = one_level_spill(depth);
     b->max_steps = (uint32_t)std::min<uint64_t>(steps, 0xFFFFFFF0ull);
     const uint32_t grid = max_trace_grid(c);
     e = hipMalloc((void**)&b->spill, (size_t)grid * KP_TRACE_BLOCK * b->spill_cap * sizeof(uint2));
@@ -1819,10 +1816,9 @@ static int batch_render(BatchState* b, const kp_render_desc* descs, uint32_t max
         for (uint64_t p = 0; p < passes; ++p)
             if ((rc = batch_enqueue_pass(b, a, tc, max_depth))) return rc;
     }
-    if ((rc = kp_synchronize(c))) return rc;
+    if ((rc = finish(c, b->ps.totals, nullptr))) return rc;
     auto t1 = std::chrono::steady_clock::now();
-    unsigned long long tot[2];
-    KP_HIP_TRY(c, hipMemcpy(tot, b->ps.totals, 16, hipMemcpyDeviceToHost));
+    const unsigned long long* tot = c->h_status->totals;
     b->stats = kp_render_stats{};
     b->stats.paths = std::min<unsigned long long>(work, (unsigned long long)passes * chunk);
     b->stats.extension_rays = tot[0];

@@ -1241,6 +1241,28 @@ __global__ void k_reset_u32(uint32_t* p, uint32_t n) {
     if (i < n) p[i] = 0u;
 }
 
+// The host's last word on a call: one kernel behind its work instead of a
+// blocking 4- to 16-byte copy per value after the wait (about 13 us each).
+__global__ void k_status(const uint32_t* err, const uint32_t* noalloc_err, const unsigned long long* totals,
+                         const uint32_t* train_records, HostStatus* out) {
+    if (threadIdx.x != 0) return;
+    HostStatus h{};
+    if (totals) {
+        h.totals[0] = totals[0];
+        h.totals[1] = totals[1];
+    }
+    if (err) h.err = *err;
+    if (noalloc_err) h.noalloc_err = *noalloc_err;
+    if (train_records) h.train_records = *train_records;
+    *out = h;
+}
+
+hipError_t launch_status(const uint32_t* err, const uint32_t* noalloc_err, const unsigned long long* totals,
+                         const uint32_t* train_records, HostStatus* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_status, dim3(1), dim3(64), 0, s, err, noalloc_err, totals, train_records, out);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------- launch --
 // Whether the launch's feeders take rays from the counter: not while first
 // chunks hold every ray (RayFeeder::init), so small launches need no clearing

@@ -221,7 +221,8 @@ int kp_occluded_host(const kp_ctx* ctx, const kp_ray* rays, uint32_t n, uint32_t
  * stream) race and must be serialised by the caller. */
 int kp_intersect_closest_noalloc(kp_ctx* ctx, const kp_ray* rays, uint32_t n, kp_hit* hits);
 /* Instrumented closest hit: same results, plus the totals of BVH8 nodes
- * visited and triangles tested (for the bytes-per-ray roofline figure). */
+ * visited and triangles tested (for the bytes-per-ray roofline figure): the
+ * triangles of the leaf children whose boxes are hit. */
 int kp_intersect_closest_counted(kp_ctx* ctx, const kp_ray* rays, uint32_t n, kp_hit* hits,
                                  int ptr_kind, uint64_t* nodes_visited,
                                  uint64_t* tris_tested);

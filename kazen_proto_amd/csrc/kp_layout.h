@@ -25,7 +25,7 @@
 //   dword 0-2  p.xyz       (low byte: e)
 //   dword 3    child_base (24 bits) | imask << 24
 //   dword 4    prim_base          read only for nodes whose leaf children
-//   dword 5-6  meta[8]            are hit
+//   dword 5-6  meta[8]            are hit (empty slots: a valid offset)
 //   dword 7    0
 //   dword 8-31 planes
 // One lane reads its node with 16-byte loads from one 128-byte line; the L1
@@ -65,6 +65,15 @@ static inline void kp_device_node(const KpNode8& n, uint32_t out[32]) {
     out[5] = meta0;
     out[6] = meta1;
     out[7] = 0u;
+    // An empty slot's meta byte: no triangles, at the offset of the leaf slots
+    // before it.  Its inverted box can be hit (the far distance is widened), and
+    // a leaf set is tested as the run from its first to its last slot.
+    uint8_t* meta = (uint8_t*)(out + 5);
+    uint32_t off = 0u;
+    for (int s = 0; s < 8; ++s) {
+        if (meta[s] == 0u) meta[s] = (uint8_t)off;
+        else if (!((n.imask >> s) & 1u)) off = (meta[s] & 31u) + (meta[s] >> 5);
+    }
 }
 
 // A leaf reference packs a triangle start (28 bits) and count-1 (3 bits).

@@ -89,3 +89,26 @@ def test_split_occlusion_with_spilled_stacks():
         assert np.array_equal(c.intersect_closest(rays[:n]).view(np.uint32),
                               c.intersect_closest_host(rays[:n]).view(np.uint32)), n
     c.close()
+
+
+@pytest.mark.parametrize("leaf_size", [1, 2, 3, 4])
+@pytest.mark.parametrize("width", [2, 5, 8])
+def test_leaf_runs(leaf_size, width):
+    """A leaf set is tested as the run of triangles from its first to its last
+    hit slot: every leaf size with narrow nodes (empty slots) and wide ones,
+    against brute force; rays from far away (boxes widened the most) and rays
+    with negative starts included."""
+    rng = np.random.default_rng(leaf_size * 10 + width)
+    tris = scenes.small_test_scene(seed=width, n_random=900)
+    rays = scenes.incoherent_rays(3000, rng)
+    rays[::4, 0:3] *= 30.0
+    rays[::4, 4:7] = -rays[::4, 0:3]
+    rays[1::5, 3] = -0.5
+    rays[2::5, 7] = 0.6
+    c = native.Context(0)
+    c.mesh_add_soup(tris)
+    c.bvh_build(leaf_size=leaf_size, node_width=width)
+    ref = oracle.closest_bruteforce(tris, rays)
+    assert np.array_equal(c.intersect_closest(rays).view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(c.occluded(rays) != 0, ref[:, 1].view(np.uint32) != 0xFFFFFFFF)
+    c.close()

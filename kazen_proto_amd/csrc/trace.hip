@@ -73,6 +73,12 @@ __device__ __forceinline__ float safe_rcp(float d) {
     return 1.0f / dd;
 }
 
+__device__ __forceinline__ float fast_rcp(float d) {
+    const float dd = fabsf(d) < 1e-20f ? copysignf(1e-20f, d) : d;
+    const float q = __builtin_amdgcn_rcpf(dd);
+    return fmaf(fmaf(-dd, q, 1.0f), q, q);
+}
+
 // Rays with a non-finite origin or direction, a zero direction or a NaN
 // interval bound miss everything (same rule as the oracle).
 __device__ __forceinline__ bool ray_valid(const float4 a, const float4 b) {
@@ -95,9 +101,18 @@ __device__ __forceinline__ void setup_ray(const float4 a, const float4 b, RayPre
     r.Sx = pick3(r.dx, r.dy, r.dz, kx) / dkz;
     r.Sy = pick3(r.dx, r.dy, r.dz, ky) / dkz;
     r.Sz = 1.0f / dkz;
-    r.ix = safe_rcp(r.dx);
-    r.iy = safe_rcp(r.dy);
-    r.iz = safe_rcp(r.dz);
+    // Reciprocals for the box tests only: the hardware estimate (1 ulp) and one
+    // Newton step, within a hair of the rounded quotient; the boxes' widening
+    // covers far more.  The estimate flushes denormal results, so a direction
+    // that large (practically never) takes the divisions.
+    r.ix = fast_rcp(r.dx);
+    r.iy = fast_rcp(r.dy);
+    r.iz = fast_rcp(r.dz);
+    if (__ballot(fmaxf(fmaxf(ax, ay), az) > 1e37f) != 0ull) {
+        r.ix = safe_rcp(r.dx);
+        r.iy = safe_rcp(r.dy);
+        r.iz = safe_rcp(r.dz);
+    }
 }
 
 // Watertight test; same operation order as the host oracle.
@@ -213,7 +228,8 @@ __device__ __forceinline__ int32_t median3(int32_t a, int32_t b, int32_t c) {
 // visit's instructions and its loads both cost time.  With seven loads (leaf
 // words only where leaves are tested), signed order keys (no clamp at zero),
 // the running second minimum as a median, and the hit kept in LDS instead of
-// four registers: 1,284 -> 1,188 us a launch.
+// four registers: 1,284 -> 1,188 us a launch (1,145 with the leaf runs below
+// and the keys formed after the slots).
 __device__ __forceinline__ void visit_node(NodeBuf nb, uint32_t idx, const RayPre& r, const NodeTest& nt,
                                            float tmax, NodeHits& h) {
     const uint32_t p = idx << 7;   // 128-byte nodes
@@ -228,7 +244,7 @@ __device__ __forceinline__ void visit_node(NodeBuf nb, uint32_t idx, const RayPr
     const float bx = (px - r.ox) * r.ix, by = (py - r.oy) * r.iy, bz = (pz - r.oz) * r.iz;
     const uint32_t imask = w0.w >> 24;
     uint32_t hit = 0u;
-    int32_t k1 = kNoKey, k2 = kNoKey;
+    float tns[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
         const float tnx = fmaf(qplane(nx, s), ax, bx);
@@ -239,11 +255,19 @@ __device__ __forceinline__ void visit_node(NodeBuf nb, uint32_t idx, const RayPr
         const float tfz = fmaf(qplane(fz, s), az, bz);
         const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, r.tmin));
         const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
-        const bool hs = tn <= fmaf(fabsf(tf), KP_FAR_EPS, tf);
-        hit |= hs ? (1u << s) : 0u;
-        // key of a hit inner child; k1 <= k2, so the second smallest of
-        // {k1, k2, key} is their median
-        const int32_t key = (hs && ((imask >> s) & 1u)) ? tkey(tn, (uint32_t)s) : kNoKey;
+        hit |= tn <= fmaf(fabsf(tf), KP_FAR_EPS, tf) ? (1u << s) : 0u;
+        tns[s] = tn;
+    }
+    // order keys of the hit inner children, the others kNoKey: the mask bit
+    // spread over the word selects (two instructions a slot; a compare and a
+    // conditional move on both conditions take four, occlusion launches 5 %).
+    // k1 <= k2, so the second smallest of {k1, k2, key} is their median.
+    int32_t k1 = kNoKey, k2 = kNoKey;
+    const uint32_t m = hit & imask;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const uint32_t mask = (uint32_t)__builtin_amdgcn_sbfe((int)m, s, 1);
+        const int32_t key = (int32_t)(((uint32_t)tkey(tns[s], (uint32_t)s) & mask) | ((uint32_t)kNoKey & ~mask));
         k2 = median3(k1, k2, key);
         k1 = min(k1, key);
     }

@@ -67,3 +67,23 @@ def test_device_nodes_give_the_same_hits(offset, scale):
     want = oracle.closest_bruteforce(tris, rays)[:, 1].view(np.uint32) != 0xFFFFFFFF
     assert np.array_equal(c.occluded(rays) != 0, want)
     c.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length", [
+    pytest.param(1e-30, marks=pytest.mark.xfail(reason="box tests clamp direction components at 1e-20, so distances "
+                                                       "in units of a shorter direction are not bracketed")),
+    1e-12, 1.0, 1e12, 9e37, 3e38])
+def test_direction_lengths(length):
+    """Directions from tiny to the largest finite ones (their reciprocals are
+    denormal), t in units of the direction's length."""
+    tris = _tris(0.0, 1.0, False)
+    rays = scenes.incoherent_rays(2049, np.random.default_rng(3))
+    with np.errstate(over="ignore"):
+        rays[:, 4:7] = (rays[:, 4:7].astype(np.float64) / np.abs(rays[:, 4:7]).max(1, keepdims=True) * length)
+    rays[::3, 3] = 0.01 / length if length < 1e30 else 1e-40
+    c = native.Context(0)
+    c.mesh_add_soup(tris)
+    c.bvh_build()
+    assert np.array_equal(c.intersect_closest(rays).view(np.uint32), oracle.closest_bruteforce(tris, rays).view(np.uint32))
+    c.close()

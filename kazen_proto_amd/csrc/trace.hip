@@ -61,7 +61,7 @@ struct RayPre {
     float ox, oy, oz, tmin, dx, dy, dz, tmax;
     float ix, iy, iz;
     float Sx, Sy, Sz;
-    int kx, ky, kz;
+    uint32_t k;   // the triangle test's axes: kx | ky << 2 | kz << 4
 };
 
 __device__ __forceinline__ float pick3(float a, float b, float c, int k) {
@@ -97,7 +97,7 @@ __device__ __forceinline__ void setup_ray(const float4 a, const float4 b, RayPre
     int ky = (kx == 2) ? 0 : kx + 1;
     const float dkz = pick3(r.dx, r.dy, r.dz, kz);
     if (dkz < 0.0f) { int t = kx; kx = ky; ky = t; }
-    r.kx = kx; r.ky = ky; r.kz = kz;
+    r.k = (uint32_t)(kx | ky << 2 | kz << 4);
     r.Sx = pick3(r.dx, r.dy, r.dz, kx) / dkz;
     r.Sy = pick3(r.dx, r.dy, r.dz, ky) / dkz;
     r.Sz = 1.0f / dkz;
@@ -119,16 +119,17 @@ __device__ __forceinline__ void setup_ray(const float4 a, const float4 b, RayPre
 __device__ __forceinline__ bool tri_test(const RayPre& r, const float4 a, const float4 b,
                                          const float4 c, float tmax_incl, float& t_out,
                                          float& u_out, float& v_out) {
+    const int kx = (int)(r.k & 3u), ky = (int)((r.k >> 2) & 3u), kz = (int)(r.k >> 4);
     const float A0 = a.x - r.ox, A1 = a.y - r.oy, A2 = a.z - r.oz;
     const float B0 = b.x - r.ox, B1 = b.y - r.oy, B2 = b.z - r.oz;
     const float C0 = c.x - r.ox, C1 = c.y - r.oy, C2 = c.z - r.oz;
-    const float Akz = pick3(A0, A1, A2, r.kz), Bkz = pick3(B0, B1, B2, r.kz), Ckz = pick3(C0, C1, C2, r.kz);
-    const float Ax = pick3(A0, A1, A2, r.kx) - r.Sx * Akz;
-    const float Ay = pick3(A0, A1, A2, r.ky) - r.Sy * Akz;
-    const float Bx = pick3(B0, B1, B2, r.kx) - r.Sx * Bkz;
-    const float By = pick3(B0, B1, B2, r.ky) - r.Sy * Bkz;
-    const float Cx = pick3(C0, C1, C2, r.kx) - r.Sx * Ckz;
-    const float Cy = pick3(C0, C1, C2, r.ky) - r.Sy * Ckz;
+    const float Akz = pick3(A0, A1, A2, kz), Bkz = pick3(B0, B1, B2, kz), Ckz = pick3(C0, C1, C2, kz);
+    const float Ax = pick3(A0, A1, A2, kx) - r.Sx * Akz;
+    const float Ay = pick3(A0, A1, A2, ky) - r.Sy * Akz;
+    const float Bx = pick3(B0, B1, B2, kx) - r.Sx * Bkz;
+    const float By = pick3(B0, B1, B2, ky) - r.Sy * Bkz;
+    const float Cx = pick3(C0, C1, C2, kx) - r.Sx * Ckz;
+    const float Cy = pick3(C0, C1, C2, ky) - r.Sy * Ckz;
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
@@ -427,15 +428,15 @@ struct RayFeeder {
         // rays (as many waves as that takes), except that a small launch whose
         // rays can be split (thin) uses one wave per SIMD with fewer rays each
         // (a grid holds five): the idle lanes then take parts of the rays from
-        // the start.  1,000 / 16,384 closest-hit rays 45 / 97 us with 64 a
-        // wave, 35 / 75 so (with every wave used 65,536 rays take 57 us where
-        // three launches are in flight, 40 so).  Occlusion rays end early and
-        // lose by it (2,000 rays 71 -> 77 us).
+        // the start.  1,000 closest-hit rays take 15.2 us with at least four
+        // rays a wave and 13.7 so, 2,000 occlusion rays 36 us with 64 a wave
+        // and 27 so (20.5 with the hand-out below).  With every wave used
+        // 65,536 rays took 57 us where three launches are in flight, 40 with
+        // one per SIMD.
         uint32_t first;
         const uint32_t per_simd = waves >= 5u ? waves / 5u : 1u;
         if (thin && n <= per_simd * 64u) {
             first = (n + per_simd - 1u) / per_simd;
-            first = first < 4u ? 4u : first;
         } else if (n <= waves * kChunk) {
             first = ((n + waves - 1u) / waves + 63u) & ~63u;
         } else {
@@ -631,9 +632,7 @@ __device__ __forceinline__ void test_leaves_wave(NodeBuf nb, const float4* __res
         o.Sx = __shfl(r.Sx, ow);
         o.Sy = __shfl(r.Sy, ow);
         o.Sz = __shfl(r.Sz, ow);
-        o.kx = __shfl(r.kx, ow);
-        o.ky = __shfl(r.ky, ow);
-        o.kz = __shfl(r.kz, ow);
+        o.k = __shfl(r.k, ow);
         const float o_best = __shfl(best_t, ow);
         const uint32_t o_off = __shfl(prim_off, ow);
         if (pos < P) {
@@ -804,10 +803,22 @@ __device__ __forceinline__ void connect_open(const TraceArgs& args, LeafLds& L, 
 //
 // Split rays (kSplit; one level): once the rays are handed out, lanes
 // whose rays are done would idle while the wave finishes its longest rays.
-// Such a lane takes the top group entry of a lane still at work and
-// traverses that group for the same ray (reloaded from the ray buffer) with
-// the donor's closest distance so far; the groups of a ray are disjoint
-// subtrees, so every triangle is still tested by exactly one lane.  A helper
+// Such a lane takes a child of the top group entry of a lane still at work
+// (the whole group where no more lanes are idle than can give) and traverses
+// it for the same ray (read from the donor's registers) with the donor's
+// closest distance so far; the children are disjoint subtrees, so every
+// triangle is still tested by exactly one lane.  A drain is bound by latency:
+// about eight passes of 5,000 to 8,000 cycles for the longest rays of a small
+// image, so a pass should spread a ray as far as there are lanes and a helper
+// start at once.  With the ray read again and set up anew, the group taken in
+// one pass and its first child visited in the next 1,000 closest-hit rays
+// took 27.6 us, 65,536 90.7, 2,000 occlusion rays 44.1 and a 160 x 120 preview
+// 343; with the ray from the donor and the first child visited at once 19.2,
+// 77.7, 36.0 and 304; with thin occlusion launches 27.0 (occlusion) and 268;
+// with single children handed out 15.2, 76.2, 22.0 and 255 (4.2 M rays lose
+// 1 % by the registers, so the axes of the triangle test share one: 1,117 us
+// before, 1,130, 1,115 now).  Two node visits between passes: 17.7, 82.3, 26.7
+// and 262.  A helper
 // merges its closest hit into its owner's slot in LDS (64-bit minimum of the
 // (distance, primitive) key, then the t, u, v of the winning key); the owner
 // writes the ray's hit once no helper of its ray is left.  The result is the
@@ -862,8 +873,8 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
     uint64_t cnt_nodes = 0, cnt_tris = 0;
     RayFeeder feed;
     // (the counted variant measures the visits a ray needs: no thin launches,
-    // which trade visits for latency, +28 % on 4,096 rays)
-    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kSplit && !kAny && !kCount);
+    // which trade visits for latency)
+    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kSplit && !kCount);
     if (kConnect) {
         set_open_count(leafl, tid, 0u);
         __builtin_amdgcn_wave_barrier();
@@ -960,33 +971,62 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                 const bool donor = can && !(__uint_as_float(e.y & 0xFFFFFF00u) > best_t);
                 const unsigned long long donors = __ballot(donor);
                 if (donors != 0ull) {
-                    const uint32_t pairs = min((uint32_t)__popcll(idle), (uint32_t)__popcll(donors));
+                    // the idle lane of rank i takes child i / donors of the
+                    // group of donor i % donors, if the group has as many (or
+                    // all of the group where every idle lane has its donor)
+                    const uint32_t n_idle = (uint32_t)__popcll(idle), n_don = (uint32_t)__popcll(donors);
                     const unsigned long long below = (1ull << lane) - 1ull;
-                    const bool give = donor && (uint32_t)__popcll(donors & below) < pairs;
+                    const float inv = __builtin_amdgcn_rcpf((float)n_don);
                     const uint32_t rank = (uint32_t)__popcll(idle & below);
-                    const bool take = ((idle >> lane) & 1ull) && rank < pairs;
-                    const int src = take ? (int)nth_set_bit(donors, rank) : (int)lane;
+                    const uint32_t kth = (uint32_t)(((float)rank + 0.5f) * inv);
+                    const bool is_idle = (idle >> lane) & 1ull;
+                    const int src = is_idle ? (int)nth_set_bit(donors, rank - kth * n_don) : (int)lane;
+                    const uint32_t mine = (uint32_t)__popcll(donors & below);
+                    const bool give = donor && mine < n_idle;
+                    const bool whole = n_idle <= n_don;
                     const uint32_t gx = __shfl(e.x, src), gy = __shfl(e.y, src);
                     const uint32_t rid = __shfl(ray_id, src);
                     const float bt = __shfl(best_t, src);
                     const uint32_t own = __shfl(role & 0xFFu, src);
+                    const bool take = is_idle && kth < (uint32_t)__popc(gy & 0xFFu);
                     if (give) {
-                        st.drop();
+                        uint32_t c = (uint32_t)(((float)(n_idle - mine - 1u) + 0.5f) * inv) + 1u;
+                        uint32_t rest = whole ? 0u : e.y & 0xFFu;
+                        while (c != 0u && rest != 0u) {
+                            rest &= rest - 1u;
+                            --c;
+                        }
+                        if (rest) st.set_top_y((e.y & 0xFFFFFF00u) | rest);
+                        else st.drop();
                         srole[tid] = role | kDonated;
                     }
+                    // the ray as its donor holds it (the others read themselves)
+                    r.ox = __shfl(r.ox, src);
+                    r.oy = __shfl(r.oy, src);
+                    r.oz = __shfl(r.oz, src);
+                    r.tmin = __shfl(r.tmin, src);
+                    r.ix = __shfl(r.ix, src);
+                    r.iy = __shfl(r.iy, src);
+                    r.iz = __shfl(r.iz, src);
+                    r.Sx = __shfl(r.Sx, src);
+                    r.Sy = __shfl(r.Sy, src);
+                    r.Sz = __shfl(r.Sz, src);
+                    r.k = __shfl(r.k, src);
                     if (take) {
                         ray_id = rid;
                         srole[tid] = own | kHelper;
-                        setup_ray(args.rays[2 * (size_t)rid], args.rays[2 * (size_t)rid + 1], r);
                         nt = node_test_setup(r);
                         best_t = bt;
                         if (!kAny) leafl.key[tid] = ~0ull;
                         occl = false;
                         pend = 0u;
-                        cur = KP_INVALID;
                         steps = 0;
                         st.sp = 0;
-                        st.push(gx, gy);   // the stack is empty: cannot overflow
+                        uint32_t pm = gy & 0xFFu;
+                        for (uint32_t k = 0u; k < kth; ++k) pm &= pm - 1u;
+                        cur = inner_child(gx & 0x00FFFFFFu, gx >> 24, (__ffs(pm) - 1u) ^ nt.oct);
+                        pm &= pm - 1u;
+                        if (whole && pm) st.push_lds(gx, (gy & 0xFFFFFF00u) | pm);
                     }
                 }
             }

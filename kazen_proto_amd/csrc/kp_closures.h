@@ -153,17 +153,22 @@ __device__ inline void beckmann_sample11(float cos_t, float u1, float u2, float&
     float b = c - (1.0f + c) * powf(1.0f - sample_x, fit);
     const float inv_sqrt_pi = 0.56418958354775628f;
     const float norm = 1.0f / (1.0f + c + inv_sqrt_pi * tan_t * expf(-cot_t * cot_t));
+    float ie = 0.0f;
+    bool found = false;
     for (int it = 0; it < 12; ++it) {
         if (!(b >= a && b <= c)) b = 0.5f * (a + c);
-        const float ie = erfinvf(b);
+        ie = erfinvf(b);
         const float value = norm * (1.0f + b + inv_sqrt_pi * tan_t * expf(-ie * ie)) - sample_x;
         const float deriv = norm * (1.0f - ie * tan_t);
-        if (fabsf(value) < 1e-6f) break;
+        if (fabsf(value) < 1e-6f) {
+            found = true;
+            break;
+        }
         if (value > 0.0f) c = b;
         else a = b;
         b -= value / deriv;
     }
-    sx = erfinvf(b);
+    sx = found ? ie : erfinvf(b);
     sy = erfinvf(2.0f * fmaxf(u2, 1e-6f) - 1.0f);
 }
 

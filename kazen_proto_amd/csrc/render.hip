@@ -529,6 +529,7 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
         uint32_t slot = 0;
         // ---- per-lane vertex set-up --------------------------------------
         bool alive = false, guided = false, recorded = false;
+        bool lit = depth == 1;   // the path's radiance is to be written
         uint32_t rec = 0;
         f3 beta = mk(0, 0, 0), beta_pre = beta, L = beta, P = beta, ng = beta, nrm = beta, wo = beta;
         Bsdf bs;
@@ -554,17 +555,15 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
             // a path starts in the queue entry of its slot, with throughput 1
             // and no radiance: the generating kernels write none of these
             slot = q;
-            float4 st0 = make_float4(1.0f, 1.0f, 1.0f, 0.0f), st1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            float4 st0 = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
             if (depth > 1) {
                 slot = qin[q];
                 st0 = a.ps.s0[slot];
-                st1 = a.ps.s1[slot];
             }
             const float4 hit = a.ps.hits[q];
             const float4 r1 = rin[2 * (size_t)q + 1];
             beta = mk(st0.x, st0.y, st0.z);
             const float prev_pdf = st0.w;
-            L = mk(st1.x, st1.y, st1.z);
             const uint32_t prim = __float_as_uint(hit.y);
             uint32_t pixel = a.seq_base + slot / a.k;
             if (a.scenes) {
@@ -585,6 +584,7 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
                     rec = (slot / a.rec_stride) * a.rec_depth;
                     // radiance gathered before the previous vertex's direction
                     // (its emission and next-event estimate included)
+                    if (depth > 1) L = ld3(a.ps.s1[slot]);
                     if (depth >= 2 && depth - 1 <= a.rec_depth)
                         a.rec_aux[2 * (size_t)(rec + depth - 2)] = make_float4(L.x, L.y, L.z, 1.0f);
                 }
@@ -623,7 +623,9 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
                         const float pl = inv_nl * (1.0f / lr.area) * (hit.x * hit.x) / (-cos_hit);
                         w = prev_pdf * prev_pdf / (prev_pdf * prev_pdf + pl * pl);
                     }
+                    if (depth > 1) L = ld3(a.ps.s1[slot]);
                     L = L + mul(beta, Le) * w;
+                    lit = true;
                 }
                 if (depth <= max_depth) {
 #pragma unroll
@@ -777,8 +779,9 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
                     }
                 }
             }
-            a.ps.s1[slot] = make_float4(L.x, L.y, L.z, 0.0f);
-            a.ps.rng[slot] = rng.state;
+            // written once and where it changes; a path that ends draws no more
+            if (lit) a.ps.s1[slot] = make_float4(L.x, L.y, L.z, 0.0f);
+            if (cont) a.ps.rng[slot] = rng.state;
         }
         uint32_t so;
         const uint32_t qo = block_append2(cont, shad, a.ps.rays_at(depth + 1), a.ps.shadows_at(depth), app_lds, so);

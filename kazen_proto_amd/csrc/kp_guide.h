@@ -167,6 +167,11 @@ __device__ inline void g_forward_chunk(const GuideNet& net, const uint32_t* xin,
     }
 }
 
+// max(x, 0), 0 for a NaN, to be rounded to bf16 (which takes every float
+// above the largest bf16, so also the bound here, to infinity).  One
+// instruction: fmaxf canonicalises x with another, 256 a wave's query.
+__device__ __forceinline__ float g_relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 3.40282347e38f); }
+
 // Rows of LDS (KP_G_ROW words each) one wave needs for g_wave_guide.
 #define KP_G_WAVE_ROWS 64
 
@@ -175,8 +180,13 @@ __device__ inline void g_forward_chunk(const GuideNet& net, const uint32_t* xin,
 // four 16-sample chunks (the per-chunk order reads them four times and waits
 // on the memory system 20 times instead of 5).  x holds the 64 bf16 input
 // rows (KP_G_ROW words each); a chunk's rows are read into registers before
-// its outputs overwrite them.  On return row s holds sample s's 32 outputs
-// as f32 (words 0..31).  Every lane of the wave must call it.
+// its outputs overwrite them.  The chunk loop is unrolled, so one chunk's
+// matrix products run while another's results are rounded and stored, and the
+// weights are read through the global address space (a generic pointer's loads
+// also wait for the LDS).  The guided shading of a 512 x 512 x 16 render: 2,063
+// us with a loop, generic loads and fmaxf, 1,930 so.  On return row s holds
+// sample s's 32 outputs as f32 (words 0..31).  Every lane of the wave must
+// call it.
 __device__ inline void g_wave_forward(const GuideNet& net, uint32_t* x) {
     const int lane = __lane_id();
     const int g = lane >> 4, r = lane & 15;
@@ -186,7 +196,8 @@ __device__ inline void g_wave_forward(const GuideNet& net, uint32_t* x) {
         const float* bias = net.params + g_layer_offset(l) + g_dim_in(l) * g_dim_out(l);
         // launder the fragment pointer per layer: loads of later layers are
         // not hoisted here (they would pin 32 registers per lane and layer)
-        const u32x4* wf = net.wf;
+        const __attribute__((address_space(1))) u32x4* wf =
+            (const __attribute__((address_space(1))) u32x4*)net.wf;
         asm volatile("" : "+s"(wf));
         u32x4 w[8];
 #pragma unroll
@@ -196,7 +207,7 @@ __device__ inline void g_wave_forward(const GuideNet& net, uint32_t* x) {
         for (int t = 0; t < ntiles; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) bv[4 * t + j] = bias[16 * t + 4 * g + j];
-#pragma unroll 1
+#pragma unroll 4
         for (int c = 0; c < 4; ++c) {
             const int row = 16 * c + r;
             const u32x4 b0 = *(const u32x4*)(x + row * KP_G_ROW + 4 * g);
@@ -213,7 +224,7 @@ __device__ inline void g_wave_forward(const GuideNet& net, uint32_t* x) {
                 for (int j = 0; j < 4; ++j) v[j] = acc[j];
                 if (l < KP_G_LAYERS - 1) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = fmaxf(v[j], 0.0f);
+                    for (int j = 0; j < 4; ++j) v[j] = g_relu(v[j]);
                     *reinterpret_cast<uint2*>(x + row * KP_G_ROW + n0 / 2) =
                         make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
                 } else {

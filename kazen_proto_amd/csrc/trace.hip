@@ -394,7 +394,7 @@ constexpr uint32_t kChunk = 256;
 constexpr uint32_t kTailChunk = 64;
 // Occlusion launches of at most this many rays per block split their rays
 // (k_occluded5<true>).
-constexpr uint32_t kSplitRays = 256;
+constexpr uint32_t kSplitRays = 512;
 
 struct RayFeeder {
     uint32_t next, end, n;
@@ -826,12 +826,11 @@ __device__ __forceinline__ void connect_open(const TraceArgs& args, LeafLds& L, 
 // without splitting.  A helper also culls with its owner's closest distance
 // once that is nearer (read at every pass of the drain phase).  An occlusion
 // ray's slot holds only whether a part of it has hit; its helpers then stop.
-// Occlusion splits in the integrator's pair launches (with 96 registers they
-// have room for it; terrain render 15.70 -> 15.55 ms, guided room 6.11 -> 6.04)
-// and, in launches of its own, up to kSplitRays rays per block: 2,000 / 65,536
-// / 200,000 rays 75 / 92 / 125 us without, 71 / 77 / 92 with; at 1,000,003 rays
-// three launches in flight take 164 us each with and 150 without (the loop has
-// five spilled registers), at 400,000 84 and 80.
+// Occlusion splits in the integrator's pair launches and, in launches of its
+// own, up to kSplitRays rays per block (in the loop it has six spilled
+// registers, the build without has none): 400,000 rays 121 us one launch at a
+// time and 67.1 with three in flight without, 111 and 66.0 with; 1,000,003 rays
+// 199 and 133 without, 189 and 137 with.
 //
 // Connect (kConnect, occlusion): instead of a flag per ray, a ray that is not
 // occluded adds its contribution to its path's radiance.  The finished rays

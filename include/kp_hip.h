@@ -249,7 +249,7 @@ int kp_bvh8_blob_occluded(const kp_bvh8_blob* b, const kp_ray* rays, uint32_t n,
 int kp_set_trace_tuning(kp_ctx* ctx, uint32_t refill_below_lanes);
 /* Tuning: at most `max_paths` paths (2^16 .. 2^28) in flight per pass of
  * kp_render / kp_render_accumulate and per chunk of kp_integrate_rays
- * (default 2^26: 13.4 GB of path state, 200 B per path). Larger passes keep
+ * (default 2^26: 13.2 GB of path state, 196 B per path). Larger passes keep
  * every bounce's launches full (a pass's later bounces hold only the paths
  * still alive); results do not depend on it. Guided renders use
  * kp_guiding_desc.pass_paths instead. */
@@ -445,11 +445,12 @@ int kp_guiding_configure(kp_ctx* ctx, const kp_guiding_desc* desc);
  * away afterwards. kp_batch_render traces descs[i].spp samples of every scene
  * i into fresh per-scene films, in passes of pass_paths paths drawn from all
  * scenes at once: each bounce is one persistent traversal launch over every
- * scene's rays. With use_graph one pass (about six launches per bounce) is
+ * scene's rays. With use_graph one pass (two launches per bounce) is
  * captured into a HIP graph once and replayed. Scene i's film equals, bit for
  * bit, kp_render of that scene alone with descs[i] (not guided).
- * kp_batch_autotune times candidate settings on `passes` passes of the
- * batch's own work, one setting at a time, and keeps the fastest. The BVH
+ * kp_batch_autotune times candidate settings on the batch's own work (the
+ * paths of `passes` passes of the largest candidate size, 2^25, for each),
+ * one setting at a time, and keeps the fastest. The BVH
  * node width is 8 in every configuration. */
 typedef struct kp_batch kp_batch;
 typedef struct {

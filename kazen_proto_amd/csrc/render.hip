@@ -17,11 +17,12 @@
 //             block and queue (same-address device atomics are the limit:
 //             one per wave made shading 3.4x slower)
 // Two launches a bounce.  A launch costs 4 to 5 us even when it has next to
-// nothing to do, and a traversal launch ends with a drain of 30 to 50 us, so
-// with closest hit, occlusion, connect, and counter clearing each launched on
-// their own (eight a bounce) a 160 x 120 preview at depth 5 took 746 us and
-// now takes 458; 256 x 256 at 16 samples 1,706 and 1,354; 1024 x 1024 at 16
-// samples of a two-million-triangle terrain at depth 8 16.59 and 15.25 ms.
+// nothing to do, and a traversal launch ends with a drain (20 us at the
+// least), so with closest hit, occlusion, connect, and counter clearing each
+// launched on their own (eight a bounce) a 160 x 120 preview at depth 5 took
+// 746 us and 458 after; 256 x 256 at 16 samples 1,706 and 1,354; 1024 x 1024
+// at 16 samples of a two-million-triangle terrain at depth 8 16.59 and 15.25
+// ms (with the steps since: 268, 1,080 and 12.6).
 // After the last bounce every pixel folds its k path radiances into the film
 // (FP32 sum with Kahan compensation, one owner per pixel, fixed order), so
 // the film does not depend on scheduling.
@@ -1939,6 +1940,7 @@ static int batch_render(BatchState* b, const kp_render_desc* descs, uint32_t max
 static int batch_autotune(BatchState* b, const kp_render_desc* descs, uint32_t passes, kp_batch_tuning* out) {
     kp_ctx* c = b->c;
     const uint32_t tb_max = std::max(c->grid_closest5, c->grid_occluded5) / (uint32_t)c->cus;
+    constexpr uint32_t kMaxPassPaths = 1u << 25;
     auto cost = [&](const kp_batch_tuning& t, double* sec_per_path) -> int {
         b->tune = t;
         uint32_t run = 0;
@@ -1947,7 +1949,13 @@ static int batch_autotune(BatchState* b, const kp_render_desc* descs, uint32_t p
                          t.trace_blocks_per_cu, t.shade_blocks_per_cu, t.refill_below);
         int rc = batch_render(b, descs, 1, &run);   // warm-up: allocation, graph capture
         if (rc) return rc;
-        if ((rc = batch_render(b, descs, passes, &run))) return rc;
+        // every candidate renders the same paths, those of `passes` passes of
+        // the largest size: the batch's first scenes may be cheaper per path
+        // than the rest, which would favour small passes (2^21 instead of 2^24
+        // on 32 uneven terrains, 1.43 instead of 2.31 G samples/s)
+        const uint64_t work = (uint64_t)passes * kMaxPassPaths;
+        const uint64_t n = (work + t.pass_paths - 1) / t.pass_paths;
+        if ((rc = batch_render(b, descs, (uint32_t)std::min<uint64_t>(n, 0xFFFFFFFFu), &run))) return rc;
         *sec_per_path = b->stats.seconds / (double)std::max<uint64_t>(1, b->stats.paths);
         if (verbose()) std::fprintf(stderr, "[kp] autotune:   %.3f ns per path\n", *sec_per_path * 1e9);
         return KP_OK;
@@ -1971,7 +1979,7 @@ static int batch_autotune(BatchState* b, const kp_render_desc* descs, uint32_t p
         }
         return KP_OK;
     };
-    if ((rc = try_values(&kp_batch_tuning::pass_paths, {1u << 21, 1u << 22, 1u << 23, 1u << 24, 1u << 25}))) return rc;
+    if ((rc = try_values(&kp_batch_tuning::pass_paths, {1u << 21, 1u << 22, 1u << 23, 1u << 24, kMaxPassPaths}))) return rc;
     if ((rc = try_values(&kp_batch_tuning::trace_blocks_per_cu, {tb_max, std::max(1u, tb_max / 2), std::max(1u, tb_max - 1)})))
         return rc;
     if ((rc = try_values(&kp_batch_tuning::refill_below, {16u, 32u, 40u, 48u, 56u}))) return rc;

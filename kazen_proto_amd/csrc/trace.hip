@@ -15,9 +15,9 @@
 //  - 128-byte nodes: seven 16-byte loads per visit (each lane loads its own
 //    near and far planes by the ray's octant; the leaf words are read only
 //    when leaf children are tested), 16-bit child boxes decoded with one fma
-//    per plane; the nearest hit inner child is visited next and the others go on the stack as one group,
-//    visited in octant order (children sit in octant slots) and culled as a
-//    group by their nearest entry distance;
+//    per plane; the nearest hit inner child is visited next and the others go
+//    on the stack as one group, visited in octant order (children sit in
+//    octant slots) and culled as a group by their nearest entry distance;
 //  - watertight ray/triangle test (Woop, Benthin, Wald 2013) with contraction
 //    disabled, so its result is bit-identical to the host oracle's;
 //  - closest hit is the smallest t, ties broken by the lowest primitive
@@ -1233,10 +1233,10 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_occluded(TraceArgs args) {
     traverse<true, false, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
-// The same traversals compiled for 5 waves per SIMD (96 registers; closest
-// hit spills one register).  Measured: the integrator's bounces on the 9.4 M
-// triangle terrain run 5 % faster, the incoherent microbench 2 % slower, so
-// only the integrator launches them.
+// The same traversals compiled for 5 waves per SIMD (96 registers; the
+// closest-hit build spills one register, the splitting occlusion build six):
+// more waves hide more of the node fetches' latency.  Launched everywhere but
+// for the counted and the allocation-free closest hit.
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_closest5(
     TraceArgs args) {
     __shared__ TraceLds lds;
@@ -1272,9 +1272,9 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
 // and a persistent launch ends with a drain (its longest rays) in which the
 // machine empties: with both in one launch the shadow blocks start on every
 // CU as its closest-hit blocks run out, so a bounce has one drain, not two
-// (30 to 50 us each: most of a bounce of a small image).  The two-level build
-// spills 94 registers and is still faster than two launches: a two-level
-// terrain render 29.5 ms before, 27.4 now.
+// (about 20 us each: most of a bounce of a small image).  The two-level build
+// spills 45 registers and is still faster than two launches: a two-level
+// terrain render 29.5 ms with two launches, 27.4 with one.
 template <bool kInst>
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace_pair(
     TraceArgs args, ShadowQueue q, uint32_t n_closest) {

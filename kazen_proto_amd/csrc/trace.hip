@@ -396,6 +396,13 @@ constexpr uint32_t kTailChunk = 64;
 // (k_occluded5<true>).
 constexpr uint32_t kSplitRays = 512;
 
+// Thin launches: up to kThinMost rays per SIMD are spread over one wave a SIMD
+// (up to kThinOne) or two, the idle lanes taking parts of them (init below).
+template <bool kAny>
+constexpr uint32_t kThinOne = kAny ? 32u : 8u;
+template <bool kAny>
+constexpr uint32_t kThinMost = kAny ? 64u : 128u;
+
 struct RayFeeder {
     uint32_t next, end, n;
     uint32_t dyn_base;  // first ray handed out by the counter (after the static chunks)
@@ -409,7 +416,7 @@ struct RayFeeder {
 
     // block / blocks: this block's index among the blocks that share the queue
     __device__ __forceinline__ void init(uint32_t* ctr, const float4* rs, const uint32_t* rts, uint32_t count,
-                                         uint32_t block, uint32_t blocks, bool thin) {
+                                         uint32_t block, uint32_t blocks, uint32_t thin_one, uint32_t thin_most) {
         counter = ctr;
         rays = rs;
         roots = rts;
@@ -426,17 +433,22 @@ struct RayFeeder {
         // first chunks hold about half the rays (256 .. 4096 per wave) and the
         // counter's chunks balance the rest.  First chunks are multiples of 64
         // rays (as many waves as that takes), except that a small launch whose
-        // rays can be split (thin) uses one wave per SIMD with fewer rays each
-        // (a grid holds five): the idle lanes then take parts of the rays from
-        // the start.  1,000 closest-hit rays take 15.2 us with at least four
-        // rays a wave and 13.7 so, 2,000 occlusion rays 36 us with 64 a wave
-        // and 27 so (20.5 with the hand-out below).  With every wave used
-        // 65,536 rays took 57 us where three launches are in flight, 40 with
-        // one per SIMD.
+        // rays can be split (thin) uses one or two waves per SIMD with fewer
+        // rays each (a grid holds five): the idle lanes then take parts of the
+        // rays from the start.  1,000 closest-hit rays take 15.2 us with at
+        // least four rays a wave and 13.7 so, 2,000 occlusion rays 36 us with
+        // 64 a wave and 27 so (20.5 with the hand-out below).  One wave per
+        // SIMD or two: 16,384 closest-hit rays 37.6 us (14.5 each where three
+        // launches are in flight) and 33.4 (14.2), 65,536 74.7 (28.3) and 61.1
+        // (26.5), 100,000 84 (64 a wave, 33.6) and 77 (33.0); occlusion 16,384
+        // 26.1 (10.6) and 24.7 (11.9), 65,536 43.4 (17.5) and 37.2 (17.0),
+        // 100,000 48 (64 a wave, 20.3) and 45.4 (20.8).  All five a SIMD take
+        // 65,536 closest-hit rays 54 us, but 36 with three launches in flight.
         uint32_t first;
         const uint32_t per_simd = waves >= 5u ? waves / 5u : 1u;
-        if (thin && n <= per_simd * 64u) {
-            first = (n + per_simd - 1u) / per_simd;
+        if (n <= per_simd * thin_most) {
+            const uint32_t used = n <= per_simd * thin_one ? per_simd : 2u * per_simd;
+            first = (n + used - 1u) / used;
         } else if (n <= waves * kChunk) {
             first = ((n + waves - 1u) / waves + 63u) & ~63u;
         } else {
@@ -873,7 +885,8 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
     RayFeeder feed;
     // (the counted variant measures the visits a ray needs: no thin launches,
     // which trade visits for latency)
-    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kSplit && !kCount);
+    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kThinOne<kAny>,
+              kSplit && !kCount ? kThinMost<kAny> : 0u);
     if (kConnect) {
         set_open_count(leafl, tid, 0u);
         __builtin_amdgcn_wave_barrier();

@@ -52,7 +52,7 @@ def test_path_counts_around_the_edges(two_level, depth):
     c.close()
 
 
-COUNTS = (1, 3, 4, 5, 63, 64, 65, 1025, 4099, 65535, 65537, 327679, 327681, 655361)
+COUNTS = (1, 3, 4, 5, 63, 64, 65, 1025, 4099, 8193, 32769, 65535, 65537, 131071, 131073, 327679, 327681, 655361)
 
 
 def test_small_launches_split_their_rays():

@@ -373,25 +373,25 @@ __device__ __forceinline__ bool bsdf_eval(const Bsdf& b, Lobe l, f3 wo, f3 wi, f
     }
     return ok;
 }
-__device__ __forceinline__ void bsdf_eval(const Bsdf& b, f3 wo, f3 wi, f3& f, float& pdf) {
+__device__ __forceinline__ bool bsdf_eval(const Bsdf& b, f3 wo, f3 wi, f3& f, float& pdf,
+                                          uint32_t pick = KP_MAX_LOBES) {
     f = mk(0.0f, 0.0f, 0.0f);
     pdf = 0.0f;
-    if (b.n) bsdf_eval(b, b.lobes[0], wo, wi, f, pdf, KP_MAX_LOBES);
+    return b.n != 0 && bsdf_eval(b, b.lobes[0], wo, wi, f, pdf, pick);
 }
 
 // Picks lobe i with probability p_i by u5, re-uses u5 rescaled inside the
-// lobe, samples it and evaluates the whole material at the sampled direction.
+// lobe and samples a direction from it (bsdf_direction: the pick and its lobe,
+// evaluated later); bsdf_sample also evaluates the whole material there.
 // One lobe or several, every closure type, the sampling and the evaluation are
 // one piece of code each.  Written out for each case the plain shading kernel
 // had 17,400 instructions and the guided one 23,400, more than the instruction
 // cache holds, and a wave of mixed closures ran most of them; now 10,500 and
-// 14,300.  A batch of eight mixed scenes 988 us before, 934 now; shading of a
+// 12,000.  A batch of eight mixed scenes 988 us before, 934 now; shading of a
 // terrain render 2,327 and 2,177 us.
-__device__ __forceinline__ bool bsdf_sample(const Bsdf& b, f3 wo, float u5, float u6, float u7, f3& wi, f3& f,
-                                            float& pdf) {
-    f = mk(0.0f, 0.0f, 0.0f);
-    pdf = 0.0f;
-    uint32_t pick = 0;
+__device__ __forceinline__ bool bsdf_direction(const Bsdf& b, f3 wo, float u5, float u6, float u7, f3& wi,
+                                               uint32_t& pick, Lobe& l) {
+    pick = 0;
     float ur = u5;
     if (b.n != 1) {
         pick = b.n;
@@ -408,8 +408,16 @@ __device__ __forceinline__ bool bsdf_sample(const Bsdf& b, f3 wo, float u5, floa
         if (pick == b.n) return false;
         ur = fmaxf(fminf((u5 - lo) / pp, 0.99999994f), 0.0f);
     }
-    const Lobe l = b.lobes[pick];
-    if (!lobe_direction(l, wo, ur, u6, u7, wi)) return false;
+    l = b.lobes[pick];
+    return lobe_direction(l, wo, ur, u6, u7, wi);
+}
+__device__ __forceinline__ bool bsdf_sample(const Bsdf& b, f3 wo, float u5, float u6, float u7, f3& wi, f3& f,
+                                            float& pdf) {
+    f = mk(0.0f, 0.0f, 0.0f);
+    pdf = 0.0f;
+    uint32_t pick;
+    Lobe l;
+    if (!bsdf_direction(b, wo, u5, u6, u7, wi, pick, l)) return false;
     const bool ok = bsdf_eval(b, b.n == 1 ? l : b.lobes[0], wo, wi, f, pdf, pick);
     return ok && (b.n == 1 || pdf > 0.0f);
 }

@@ -548,6 +548,7 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
         bool bs_ok = false;
         f3 bs_wi = beta, bs_f = beta;
         float bs_pdf = 0.0f;
+        uint32_t bs_pick = KP_MAX_LOBES;
         bool use_guide = false;
         uint32_t max_depth = a.max_depth, rr_depth = a.rr_depth, n_lights = a.n_lights, light_first = 0,
                  root = 0;
@@ -691,7 +692,12 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
                     }
                     if (alive) {
                         if constexpr (kGuided) use_guide = guided && !(u[8] < a.bsdf_frac);
-                        if (!use_guide) bs_ok = bsdf_sample(bs, wo, u[5], u[6], u[7], bs_wi, bs_f, bs_pdf);
+                        if constexpr (kGuided) {
+                            Lobe l;
+                            if (!use_guide) bs_ok = bsdf_direction(bs, wo, u[5], u[6], u[7], bs_wi, bs_pick, l);
+                        } else {
+                            bs_ok = bsdf_sample(bs, wo, u[5], u[6], u[7], bs_wi, bs_f, bs_pdf);
+                        }
                     }
                 }
             }
@@ -745,14 +751,22 @@ __global__ __launch_bounds__(256, kGuided ? 3 : 4) void k_shade(RenderArgs a, in
                 f3 wi = bs_wi, f = bs_f;
                 float pdf = bs_pdf;
                 bool ok = bs_ok;
-                if (use_guide) {
-                    wi = fr.to_local(mk(ga.dx, ga.dy, ga.dz));
-                    float pdf_bsdf;
-                    bsdf_eval(bs, wo, wi, f, pdf_bsdf);
-                    pdf = a.bsdf_frac * pdf_bsdf + (1.0f - a.bsdf_frac) * ga.pdf_b;
-                    ok = !is_zero(f) && pdf > 0.0f;
-                } else if (guided && ok) {
-                    pdf = a.bsdf_frac * bs_pdf + (1.0f - a.bsdf_frac) * ga.pdf_b;
+                if constexpr (kGuided) {
+                    // one evaluation for sampled and guided directions, as lanes
+                    // of either kind share a wave (with one for each, the sampled
+                    // ones before the query, the guided room's shading took
+                    // 1,946 us a render and 1,880 so)
+                    if (use_guide) wi = fr.to_local(mk(ga.dx, ga.dy, ga.dz));
+                    if (use_guide || ok) {
+                        const bool drawn = bsdf_eval(bs, wo, wi, f, pdf, bs_pick);
+                        if (use_guide) {
+                            pdf = a.bsdf_frac * pdf + (1.0f - a.bsdf_frac) * ga.pdf_b;
+                            ok = !is_zero(f) && pdf > 0.0f;
+                        } else {
+                            ok = drawn && (bs.n == 1 || pdf > 0.0f);
+                            if (guided) pdf = a.bsdf_frac * pdf + (1.0f - a.bsdf_frac) * ga.pdf_b;
+                        }
+                    }
                 }
                 if (ok) {
                     beta = mul(beta, f) * (fabsf(wi.y) / pdf);

@@ -416,7 +416,8 @@ struct RayFeeder {
 
     // block / blocks: this block's index among the blocks that share the queue
     __device__ __forceinline__ void init(uint32_t* ctr, const float4* rs, const uint32_t* rts, uint32_t count,
-                                         uint32_t block, uint32_t blocks, uint32_t thin_one, uint32_t thin_most) {
+                                         uint32_t block, uint32_t blocks, uint32_t thin_one, uint32_t thin_most,
+                                         bool even) {
         counter = ctr;
         rays = rs;
         roots = rts;
@@ -444,13 +445,19 @@ struct RayFeeder {
         // 26.1 (10.6) and 24.7 (11.9), 65,536 43.4 (17.5) and 37.2 (17.0),
         // 100,000 48 (64 a wave, 20.3) and 45.4 (20.8).  All five a SIMD take
         // 65,536 closest-hit rays 54 us, but 36 with three launches in flight.
+        // Multiples of 64 leave some waves without rays, which costs the launch
+        // and helps others in flight (800,000 rays 278 and 184 us; evenly dealt
+        // 248 and 191).  The first launch of a pass (even), whose camera rays
+        // take about the same time each, deals them evenly: a batch of eight
+        // scenes 931 -> 893 us; later bounces gain nothing by it.
         uint32_t first;
         const uint32_t per_simd = waves >= 5u ? waves / 5u : 1u;
         if (n <= per_simd * thin_most) {
             const uint32_t used = n <= per_simd * thin_one ? per_simd : 2u * per_simd;
             first = (n + used - 1u) / used;
         } else if (n <= waves * kChunk) {
-            first = ((n + waves - 1u) / waves + 63u) & ~63u;
+            first = (n + waves - 1u) / waves;
+            first = even ? max(first, 64u) : (first + 63u) & ~63u;
         } else {
             first = (n / (2u * waves)) & ~63u;
             first = first < kChunk ? kChunk : (first > 4096u ? 4096u : first);
@@ -886,7 +893,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
     // (the counted variant measures the visits a ray needs: no thin launches,
     // which trade visits for latency)
     feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kThinOne<kAny>,
-              kSplit && !kCount ? kThinMost<kAny> : 0u);
+              kSplit && !kCount ? kThinMost<kAny> : 0u, args.n_dev != nullptr && blocks == gridDim.x);
     if (kConnect) {
         set_open_count(leafl, tid, 0u);
         __builtin_amdgcn_wave_barrier();

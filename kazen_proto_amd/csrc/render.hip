@@ -22,7 +22,7 @@
 // launched on their own (eight a bounce) a 160 x 120 preview at depth 5 took
 // 746 us and 458 after; 256 x 256 at 16 samples 1,706 and 1,354; 1024 x 1024
 // at 16 samples of a two-million-triangle terrain at depth 8 16.59 and 15.25
-// ms (with the steps since: 268, 1,080 and 12.6).
+// ms (with the steps since: 271, 1,057 and 12.5).
 // After the last bounce every pixel folds its k path radiances into the film
 // (FP32 sum with Kahan compensation, one owner per pixel, fixed order), so
 // the film does not depend on scheduling.

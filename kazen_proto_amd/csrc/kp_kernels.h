@@ -30,7 +30,7 @@ struct TraceArgs {
     uint32_t spill_blocks;  // blocks of KP_TRACE_BLOCK lanes the spill area covers (launch grid limit)
     uint32_t refill_below;  // refill a wave once fewer lanes than this are busy
     uint32_t* err;          // bit0 stack overflow, bit1 step limit
-    uint32_t max_steps;     // per-ray step limit (> any legitimate traversal)
+    uint32_t max_steps;     // node visits of one ray (> any legitimate traversal)
     unsigned long long* counters;   // [nodes visited, triangles tested]
     const uint32_t* roots;  // if set, root node of each ray (batched scenes); else node 0
     // two-level traversal (instances): nodes [0, n_tlas) are the top level,

@@ -1067,6 +1067,10 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                     if (kCount) cnt_nodes++;
                     const uint32_t vis = cur;
                     cur = KP_INVALID;
+                    // (steps are node visits: a lane whose postponed leaves
+                    // wait for the wave's test may wait for any number of the
+                    // wave's other rays)
+                    ++steps;
                     if (kInst && h.leaves && vis < args.n_tlas) {
                         // top-level leaves: push every instance they name
                         uint32_t lm = h.leaves;
@@ -1189,7 +1193,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
                     pend = 0u;
                 }
                 bool done = busy && (fault || (kAny && occl) || (cur == KP_INVALID && pend == 0u && st.sp == 0));
-                if (busy && !done && ++steps > args.max_steps) {
+                if (busy && !done && steps > args.max_steps) {
                     atomicOr(args.err, 2u);
                     done = true;
                 }

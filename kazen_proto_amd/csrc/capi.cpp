@@ -55,6 +55,7 @@ TraceArgs trace_base(kp_ctx* c) {
     a.spill = c->d_spill;
     a.spill_cap = c->spill_area;
     a.spill_blocks = (uint32_t)(c->spill_lanes / KP_TRACE_BLOCK);
+    a.simds = 4u * (uint32_t)c->cus;
     a.refill_below = c->refill_below;
     a.counters = c->d_counters;
     a.max_steps = c->max_steps;

@@ -49,6 +49,7 @@ struct TraceArgs {
     // contribution and path slot, per slot the radiance it is added to
     const float4* scontrib;
     float4* radiance;
+    uint32_t simds;         // of the device (kp_feed.h)
 };
 
 // The shadow queue of a pair launch (the rest as in its TraceArgs).

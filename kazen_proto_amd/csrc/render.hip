@@ -1890,6 +1890,7 @@ static int batch_render(BatchState* b, const kp_render_desc* descs, uint32_t max
     tc.base.spill_blocks = max_trace_grid(c);
     tc.base.five_waves = 1;   // the integrator's 5-wave traversal kernels
     tc.base.spill_cap = b->spill_cap;
+    tc.base.simds = 4u * (uint32_t)c->cus;
     tc.base.refill_below = b->tune.refill_below;
     tc.base.max_steps = b->max_steps;
     tc.base.counters = c->d_counters;

@@ -26,6 +26,7 @@
 
 #include <mutex>
 
+#include "kp_feed.h"
 #include "kp_kernels.h"
 #include "kp_layout.h"
 
@@ -390,19 +391,6 @@ constexpr int kStack = KP_TRACE_STACK;
 // and hands them to its lanes from a wave-uniform cursor; every lane keeps
 // its next ray prefetched in registers, so replacing a finished ray costs no
 // memory round trip.  All members except the prefetch are wave-uniform.
-constexpr uint32_t kChunk = 256;
-constexpr uint32_t kTailChunk = 64;
-// Occlusion launches of at most this many rays per block split their rays
-// (k_occluded5<true>).
-constexpr uint32_t kSplitRays = 512;
-
-// Thin launches: up to kThinMost rays per SIMD are spread over one wave a SIMD
-// (up to kThinOne) or two, the idle lanes taking parts of them (init below).
-template <bool kAny>
-constexpr uint32_t kThinOne = kAny ? 32u : 8u;
-template <bool kAny>
-constexpr uint32_t kThinMost = kAny ? 64u : 128u;
-
 struct RayFeeder {
     uint32_t next, end, n;
     uint32_t dyn_base;  // first ray handed out by the counter (after the static chunks)
@@ -416,8 +404,8 @@ struct RayFeeder {
 
     // block / blocks: this block's index among the blocks that share the queue
     __device__ __forceinline__ void init(uint32_t* ctr, const float4* rs, const uint32_t* rts, uint32_t count,
-                                         uint32_t block, uint32_t blocks, uint32_t thin_one, uint32_t thin_most,
-                                         bool even) {
+                                         uint32_t block, uint32_t blocks, uint32_t simds, uint32_t thin_one,
+                                         uint32_t thin_most, bool even) {
         counter = ctr;
         rays = rs;
         roots = rts;
@@ -430,38 +418,7 @@ struct RayFeeder {
         // and a wave whose first chunk lies beyond the rays has none.
         waves = blocks * (KP_TRACE_BLOCK / 64);
         const uint32_t wave = block * (KP_TRACE_BLOCK / 64) + (threadIdx.x >> 6);
-        // up to kChunk rays per wave: every ray in a first chunk; more: the
-        // first chunks hold about half the rays (256 .. 4096 per wave) and the
-        // counter's chunks balance the rest.  First chunks are multiples of 64
-        // rays (as many waves as that takes), except that a small launch whose
-        // rays can be split (thin) uses one or two waves per SIMD with fewer
-        // rays each (a grid holds five): the idle lanes then take parts of the
-        // rays from the start.  1,000 closest-hit rays take 15.2 us with at
-        // least four rays a wave and 13.7 so, 2,000 occlusion rays 36 us with
-        // 64 a wave and 27 so (20.5 with the hand-out below).  One wave per
-        // SIMD or two: 16,384 closest-hit rays 37.6 us (14.5 each where three
-        // launches are in flight) and 33.4 (14.2), 65,536 74.7 (28.3) and 61.1
-        // (26.5), 100,000 84 (64 a wave, 33.6) and 77 (33.0); occlusion 16,384
-        // 26.1 (10.6) and 24.7 (11.9), 65,536 43.4 (17.5) and 37.2 (17.0),
-        // 100,000 48 (64 a wave, 20.3) and 45.4 (20.8).  All five a SIMD take
-        // 65,536 closest-hit rays 54 us, but 36 with three launches in flight.
-        // Multiples of 64 leave some waves without rays, which costs the launch
-        // and helps others in flight (800,000 rays 278 and 184 us; evenly dealt
-        // 248 and 191).  The first launch of a pass (even), whose camera rays
-        // take about the same time each, deals them evenly: a batch of eight
-        // scenes 931 -> 893 us; later bounces gain nothing by it.
-        uint32_t first;
-        const uint32_t per_simd = waves >= 5u ? waves / 5u : 1u;
-        if (n <= per_simd * thin_most) {
-            const uint32_t used = n <= per_simd * thin_one ? per_simd : 2u * per_simd;
-            first = (n + used - 1u) / used;
-        } else if (n <= waves * kChunk) {
-            first = (n + waves - 1u) / waves;
-            first = even ? max(first, 64u) : (first + 63u) & ~63u;
-        } else {
-            first = (n / (2u * waves)) & ~63u;
-            first = first < kChunk ? kChunk : (first > 4096u ? 4096u : first);
-        }
+        const uint32_t first = first_chunk(n, waves, simds, thin_one, thin_most, even);
         dyn_base = waves * first;
         next = wave * first;
         if (next < n) {
@@ -892,7 +849,7 @@ __device__ __forceinline__ void traverse(const TraceArgs& args, TraceLds& S, uin
     RayFeeder feed;
     // (the counted variant measures the visits a ray needs: no thin launches,
     // which trade visits for latency)
-    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, kThinOne<kAny>,
+    feed.init(args.counter, args.rays, args.roots, n_rays, block, blocks, args.simds, kThinOne<kAny>,
               kSplit && !kCount ? kThinMost<kAny> : 0u, args.n_dev != nullptr && blocks == gridDim.x);
     if (kConnect) {
         set_open_count(leafl, tid, 0u);
@@ -1374,7 +1331,7 @@ hipError_t launch_status(const uint32_t* err, const uint32_t* noalloc_err, const
 // launch before them (5 us; 1,000 rays with three launches in flight 11.3 us
 // a launch with it).
 static bool uses_counter(const TraceArgs& a, uint32_t grid) {
-    return a.n_dev || (uint64_t)a.n > (uint64_t)grid * (KP_TRACE_BLOCK / 64) * kChunk;
+    return a.n_dev || !first_chunks_hold_all(a.n, grid * (KP_TRACE_BLOCK / 64));
 }
 
 hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool reset, hipStream_t s) {

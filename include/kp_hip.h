@@ -91,8 +91,8 @@ typedef struct {
     uint64_t bvh_bytes;        /* nodes + triangle records on the device */
     uint32_t max_depth;        /* BVH8 levels */
     uint32_t spill_entries;    /* per-lane stack spill capacity */
-    uint32_t grid_closest;     /* persistent blocks per launch */
-    uint32_t grid_occluded;
+    uint32_t grid_closest;     /* persistent blocks of a kp_intersect_closest launch */
+    uint32_t grid_occluded;    /* the same of a kp_occluded launch */
     double build_seconds;      /* host BVH build wall time */
     uint32_t device_cus;
     uint32_t two_level;        /* 1: instances traversed two-level; 0: one-level (baked) */

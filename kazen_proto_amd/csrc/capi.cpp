@@ -42,7 +42,7 @@ int ensure_buffer(kp_ctx* c, void** buf, size_t* cap, size_t bytes) {
 // Largest grid of any traversal launch (the integrator's pair launches hold
 // both 5-wave grids): the spill area has one slice per lane of it.
 uint32_t max_trace_grid(const kp_ctx* c) {
-    return std::max(std::max(c->grid_closest, c->grid_occluded), c->grid_closest5 + c->grid_occluded5);
+    return std::max(c->grid_closest, c->grid_closest5 + c->grid_occluded5);
 }
 
 TraceArgs trace_base(kp_ctx* c) {
@@ -105,7 +105,6 @@ int trace_occluded_dev(kp_ctx* c, const float4* rays, uint32_t n, uint32_t* out)
     a.rays = rays;
     a.occl = out;
     a.n = n;
-    a.five_waves = 1u;   // the 5-wave builds, as the integrator's shadow rays
     hipError_t e = launch_occluded(a, c->grid_occluded5, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "occlusion launch");
     return KP_OK;
@@ -397,10 +396,9 @@ int kp_create(kp_ctx** out, int device) {
         return bail(e, "alloc");
     if ((e = hipMemsetAsync(c->d_counters, 0, 64, c->stream)) != hipSuccess) return bail(e, "memset");
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return bail(e, "memset");
-    int bc = 0, bo = 0;
-    if ((e = kp::trace_occupancy(&bc, &bo)) != hipSuccess) return bail(e, "occupancy");
+    int bc = 0;
+    if ((e = kp::trace_occupancy(&bc)) != hipSuccess) return bail(e, "occupancy");
     c->grid_closest = (uint32_t)(c->cus * (bc > 0 ? bc : 1));
-    c->grid_occluded = (uint32_t)(c->cus * (bo > 0 ? bo : 1));
     int b5c = 0, b5o = 0;
     if ((e = kp::trace_occupancy_five(&b5c, &b5o)) != hipSuccess) return bail(e, "occupancy");
     c->grid_closest5 = (uint32_t)(c->cus * (b5c > 0 ? b5c : 1));
@@ -855,8 +853,8 @@ int kp_get_stats(kp_ctx* c, kp_stats* s) {
                    (c->two_level ? (uint64_t)c->inst_blas.size() * 68u : 0u);
     s->max_depth = c->max_depth;
     s->spill_entries = c->spill_cap;
-    s->grid_closest = c->grid_closest;
-    s->grid_occluded = c->grid_occluded;
+    s->grid_closest = c->grid_closest5;
+    s->grid_occluded = c->grid_occluded5;
     s->build_seconds = c->build_seconds;
     s->device_cus = (uint32_t)c->cus;
     s->two_level = c->two_level ? 1u : 0u;

@@ -58,9 +58,9 @@ struct kp_ctx {
     uint32_t spill_cap = 0;      // entries per lane: reported, and laid out in the static scratch
     uint32_t spill_area = 0;     // entries per lane of d_spill
     size_t spill_lanes = 0;
-    uint32_t grid_closest = 0, grid_occluded = 0;
+    uint32_t grid_closest = 0;                            // the 4-wave closest hit (counted, allocation-free)
     uint32_t shade_blocks = 0, shade_blocks_guided = 0;   // resident blocks of k_shade, whole device
-    uint32_t grid_closest5 = 0, grid_occluded5 = 0;       // the integrator's 5-wave traversal kernels
+    uint32_t grid_closest5 = 0, grid_occluded5 = 0;       // the 5-wave traversal kernels (all other launches)
     uint32_t refill_below = 40;   // measured best for incoherent rays (leaf 4; 36..60 swept)
     uint32_t pass_paths = 1u << 26;   // paths per pass of the integrator (measured: larger is faster)
     uint32_t max_steps = 64;

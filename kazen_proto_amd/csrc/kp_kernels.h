@@ -23,7 +23,7 @@ struct TraceArgs {
     float4* hits;           // closest: {t, prim bits, u, v}
     uint32_t* occl;         // occluded: 0/1 per ray
     uint32_t n;             // ray count
-    const uint32_t* n_dev;  // if set, the ray count is read from device memory
+    const uint32_t* n_dev;  // if set, the ray count is read from device memory (not by launch_occluded)
     uint32_t* counter;      // work counter (reset by the launcher)
     uint2* spill;           // per-lane stack spill area
     uint32_t spill_cap;     // entries per lane
@@ -42,8 +42,8 @@ struct TraceArgs {
     const uint32_t* tlas_inst;
     uint32_t n_tlas;
     uint32_t world_root;
-    // one-level closest / occluded launches of the integrator: the kernels
-    // compiled for 5 waves per SIMD (96 registers) instead of 4
+    // closest hit (launch_closest): the kernels compiled for 5 waves per SIMD
+    // (96 registers) instead of 4; occlusion and pair launches have no others
     uint32_t five_waves;
     // connecting occlusion (set inside the pair kernel): per ray its
     // contribution and path slot, per slot the radiance it is added to
@@ -69,7 +69,8 @@ hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool re
 hipError_t launch_pair(const TraceArgs& a, const ShadowQueue& q, uint32_t grid_closest, uint32_t grid_occluded,
                        hipStream_t s);
 hipError_t launch_occluded(const TraceArgs& a, uint32_t grid, hipStream_t s);
-hipError_t trace_occupancy(int* blocks_per_cu_closest, int* blocks_per_cu_occluded);
+// Blocks per CU of the 4-wave closest hit, and of the 5-wave builds.
+hipError_t trace_occupancy(int* blocks_per_cu_closest);
 hipError_t trace_occupancy_five(int* blocks_per_cu_closest, int* blocks_per_cu_occluded);
 hipError_t shade_occupancy(int* blocks_per_cu_plain, int* blocks_per_cu_guided);
 // What the host reads after waiting for the stream (page-locked memory the

@@ -1,10 +1,11 @@
 // BVH8 traversal kernels of the HIP intersector (gfx950, wave64).
 //
-// k_closest  : closest hit, replaces EmbreeAccel::intersect
-//              (reference src/core/accel.cpp:348-407; interface
-//              HitableInterface::intersect, src/core/hitable.h:12-13)
-// k_occluded : any hit in [tmin, tmax], replaces HitableInterface::occluded
-//              (src/core/hitable.h:15-33)
+// k_closest*    : closest hit, replaces EmbreeAccel::intersect
+//                 (reference src/core/accel.cpp:348-407; interface
+//                 HitableInterface::intersect, src/core/hitable.h:12-13)
+// k_occluded*   : any hit in [tmin, tmax], replaces HitableInterface::occluded
+//                 (src/core/hitable.h:15-33)
+// k_trace_pair  : both, for one bounce of the integrator
 //
 // Design:
 //  - persistent lanes: every lane owns one ray at a time; finished lanes are
@@ -1209,15 +1210,10 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_closest(TraceArgs args) {
     traverse<false, kCount, false>(args, lds, blockIdx.x, gridDim.x);
 }
 
-__global__ __launch_bounds__(KP_TRACE_BLOCK) void k_occluded(TraceArgs args) {
-    __shared__ TraceLds lds;
-    traverse<true, false, false>(args, lds, blockIdx.x, gridDim.x);
-}
-
-// The same traversals compiled for 5 waves per SIMD (96 registers; the
-// closest-hit build spills one register, the splitting occlusion build six):
-// more waves hide more of the node fetches' latency.  Launched everywhere but
-// for the counted and the allocation-free closest hit.
+// The traversals compiled for 5 waves per SIMD (96 registers; the closest-hit
+// build spills one register, the splitting occlusion build seven): more waves
+// hide more of the node fetches' latency.  Launched everywhere but for the
+// counted and the allocation-free closest hit.
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_closest5(
     TraceArgs args) {
     __shared__ TraceLds lds;
@@ -1231,8 +1227,8 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
     traverse<true, false, false, false, kSplit>(args, lds, blockIdx.x, gridDim.x);
 }
 
-// The two-level traversals compiled for 5 waves per SIMD (96 registers, 44 B
-// of spill per lane; 31 KB of LDS per block, so 5 blocks fit a CU): the
+// The two-level traversals compiled for 5 waves per SIMD (96 registers,
+// spilling 24 and 44 B per lane; 31 KB of LDS per block, so 5 blocks fit a CU): the
 // integrator's two-level render of C3's terrain runs 2.3 % faster than with
 // the 4-wave build.
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_closest_inst5(
@@ -1254,7 +1250,7 @@ __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
 // machine empties: with both in one launch the shadow blocks start on every
 // CU as its closest-hit blocks run out, so a bounce has one drain, not two
 // (about 20 us each: most of a bounce of a small image).  The two-level build
-// spills 45 registers and is still faster than two launches: a two-level
+// spills 30 registers and is still faster than two launches: a two-level
 // terrain render 29.5 ms with two launches, 27.4 with one.
 template <bool kInst>
 __global__ __launch_bounds__(KP_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(5))) void k_trace_pair(
@@ -1277,11 +1273,6 @@ template <bool kCount>
 __global__ __launch_bounds__(KP_TRACE_BLOCK) void k_closest_inst(TraceArgs args) {
     __shared__ TraceLds lds;
     traverse<false, kCount, true>(args, lds, blockIdx.x, gridDim.x);
-}
-
-__global__ __launch_bounds__(KP_TRACE_BLOCK) void k_occluded_inst(TraceArgs args) {
-    __shared__ TraceLds lds;
-    traverse<true, false, true>(args, lds, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(256) void k_copy16(uint4* __restrict__ dst, const uint4* __restrict__ src,
@@ -1352,12 +1343,10 @@ hipError_t launch_closest(const TraceArgs& a, uint32_t grid, bool count, bool re
 hipError_t launch_occluded(const TraceArgs& a, uint32_t grid, hipStream_t s) {
     if (grid == 0 || grid > a.spill_blocks) return hipErrorInvalidValue;   // lanes without a spill slice
     if (uses_counter(a, grid)) hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(64), 0, s, a.counter, 1u);
-    if (a.insts && a.five_waves) hipLaunchKernelGGL(k_occluded_inst5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
-    else if (a.insts) hipLaunchKernelGGL(k_occluded_inst, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
-    else if (a.five_waves && !a.n_dev && (uint64_t)a.n <= (uint64_t)grid * kSplitRays)
+    if (a.insts) hipLaunchKernelGGL(k_occluded_inst5, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
+    else if ((uint64_t)a.n <= (uint64_t)grid * kSplitRays)
         hipLaunchKernelGGL(k_occluded5<true>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
-    else if (a.five_waves) hipLaunchKernelGGL(k_occluded5<false>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
-    else hipLaunchKernelGGL(k_occluded, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
+    else hipLaunchKernelGGL(k_occluded5<false>, dim3(grid), dim3(KP_TRACE_BLOCK), 0, s, a);
     return hipGetLastError();
 }
 
@@ -1371,12 +1360,8 @@ hipError_t launch_pair(const TraceArgs& a, const ShadowQueue& q, uint32_t grid_c
     return hipGetLastError();
 }
 
-hipError_t trace_occupancy(int* blocks_per_cu_closest, int* blocks_per_cu_occluded) {
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu_closest,
-                                                                k_closest<false>, KP_TRACE_BLOCK, 0);
-    if (e != hipSuccess) return e;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu_occluded, k_occluded,
-                                                        KP_TRACE_BLOCK, 0);
+hipError_t trace_occupancy(int* blocks_per_cu_closest) {
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu_closest, k_closest<false>, KP_TRACE_BLOCK, 0);
 }
 
 // Blocks per CU of the 5-wave builds: the smaller of the one-level and the

@@ -41,7 +41,9 @@ typedef struct kp_ctx kp_ctx;
 
 /* Ray: origin, tmin, direction, tmax (32 bytes). Directions need not be
  * normalised; t is measured in units of |d|. Valid hits have t in
- * [tmin, tmax]. Mirrors Ray (reference src/core/ray.h:10-45) without the
+ * [tmin, tmax]. The box tests take a direction component nearer to zero than
+ * 1e-20 as 1e-20, so the direction's largest component should exceed that by
+ * far (1e-12 is tested): hits of a shorter direction may be missed. Mirrors Ray (reference src/core/ray.h:10-45) without the
  * differentials and time. */
 typedef struct {
     float ox, oy, oz, tmin;
@@ -90,7 +92,11 @@ typedef struct {
     uint64_t n_bvh2_nodes;
     uint64_t bvh_bytes;        /* nodes + triangle records on the device */
     uint32_t max_depth;        /* BVH8 levels */
-    uint32_t spill_entries;    /* per-lane stack spill capacity */
+    uint32_t spill_entries;    /* stack entries per lane that kp_intersect_closest_noalloc lays out in
+                                * its scratch (7 a level + 8; two-level 8 a top level + 7 a prototype
+                                * level + 16). The other launches' stacks spill into what a lane can
+                                * need at most: one entry a level + 2 (8 a top level + 1 a prototype
+                                * level + 16). */
     uint32_t grid_closest;     /* persistent blocks of a kp_intersect_closest launch */
     uint32_t grid_occluded;    /* the same of a kp_occluded launch */
     double build_seconds;      /* host BVH build wall time */
@@ -455,7 +461,7 @@ int kp_guiding_configure(kp_ctx* ctx, const kp_guiding_desc* desc);
 typedef struct kp_batch kp_batch;
 typedef struct {
     uint32_t pass_paths;           /* paths in flight per pass (queue size), 256 .. 2^25 */
-    uint32_t shade_blocks_per_cu;  /* 256-thread shade / connect blocks per CU */
+    uint32_t shade_blocks_per_cu;  /* 256-thread shade blocks per CU */
     uint32_t trace_blocks_per_cu;  /* persistent traversal blocks per CU (occupancy) */
     uint32_t refill_below;         /* traversal wave refill threshold, lanes 1..64 */
     uint32_t use_graph;            /* replay a captured pass graph */

@@ -311,12 +311,12 @@ static int build_two_level(kp_ctx* c, const BuildOptions& bo, double* seconds) {
     *seconds = std::chrono::duration<double>(t1 - t0).count();
     if (c->device >= 0) KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
     free_bvh(c);
-    // Stack bound: the top-level marker, at most 8 entries
-    // per top-level node on the path (instance entries and one group), the
-    // return marker, 7 per prototype level.
+    // Stack bound: the top-level marker, at most 8 entries per top-level node
+    // on the path (instance entries and one group), the return marker, and per
+    // prototype level one group (7 single children in the static scratch).
     // Postponed leaves need no stack entries.
     c->spill_cap = 8u * top.max_depth + 7u * max_unit_depth + 16u;
-    c->spill_area = 8u * top.max_depth + max_unit_depth + 16u;   // one group per prototype level
+    c->spill_area = 8u * top.max_depth + max_unit_depth + 16u;
     if (c->device >= 0) {
         const size_t tbytes = tris.size() * sizeof(float);
         const int urc = upload_nodes(c, nodes);
@@ -658,8 +658,8 @@ int kp_instance_get(kp_ctx* c, uint32_t instance_id, uint32_t* blas_id, float* o
 static int install_one_level(kp_ctx* c, kp::Bvh8Host& h, uint32_t n_all, uint32_t n_world, uint32_t width) {
     if (c->device >= 0) KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
     kp::free_bvh(c);
-    // Worst-case stack: 7 pushes per level below the root, plus slack; the
-    // top KP_TRACE_STACK entries live in LDS.
+    // 7 single children a level, plus slack, in the static scratch; one group
+    // entry a level in the context's own area.
     c->spill_cap = 7u * h.max_depth + 8u;
     c->spill_area = kp::one_level_spill(h.max_depth);
     if (c->device >= 0) {

@@ -327,9 +327,12 @@ __device__ __forceinline__ void g_grad_store(float* part, int wave, int lane, co
 // keeps them in registers; with the samples split, every wave read all 64
 // fragments (64 KB) for every 16 samples.  Operands with samples along k come
 // from transposing LDS reads instead of eight 16-bit reads each.  At 262,144
-// samples: 197 us before, 119 now (27.4 GFLOP of algorithmic work, 230 TFLOP/s); what
-// is left is the chain of about 14 barriers a group and the output gradient's
-// transcendentals at two waves per SIMD.
+// samples: 197 us before, 119 now.  The step needs 98,304 operations a sample
+// (forward 34,816, weight gradients the same, input gradients of layers 1-4
+// 28,672), 25.8 GFLOP, so 217 TFLOP/s; issued are 432 products a group, 29.0
+// GFLOP (layer 0 padded to 64 inputs, bias gradients as products with ones).
+// What is left is the chain of about 14 barriers a group and the output
+// gradient's transcendentals at two waves per SIMD.
 __global__ __launch_bounds__(256, 2) void k_guide_train(GuideNet net, const float* __restrict__ in6,
                                                         const float* __restrict__ dirs,
                                                         const float* __restrict__ weights,

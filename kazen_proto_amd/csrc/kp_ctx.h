@@ -55,8 +55,11 @@ struct kp_ctx {
     uint4* d_nodes = nullptr;
     float4* d_tris = nullptr;
     uint2* d_spill = nullptr;
-    uint32_t spill_cap = 0;      // entries per lane: reported, and laid out in the static scratch
-    uint32_t spill_area = 0;     // entries per lane of d_spill
+    // Stack entries per lane: laid out in the static scratch and reported (the
+    // bound of a stack of single children, kept so that the same BVHs fit the
+    // scratch), and in d_spill (what group entries can need).
+    uint32_t spill_cap = 0;
+    uint32_t spill_area = 0;
     size_t spill_lanes = 0;
     uint32_t grid_closest = 0;                            // the 4-wave closest hit (counted, allocation-free)
     uint32_t shade_blocks = 0, shade_blocks_guided = 0;   // resident blocks of k_shade, whole device

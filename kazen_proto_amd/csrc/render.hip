@@ -1950,8 +1950,10 @@ static int batch_render(BatchState* b, const kp_render_desc* descs, uint32_t max
 }
 
 // Coordinate descent over the launch settings, one setting at a time, each
-// candidate timed over `passes` passes of the batch's own work (seconds per
-// path, the first pass of each candidate is a warm-up).
+// candidate timed over the same paths of the batch's own work, those of
+// `passes` passes of the largest candidate size (seconds per path; one pass
+// before them is a warm-up).  A small pass size then renders up to 16 times
+// `passes` passes.
 static int batch_autotune(BatchState* b, const kp_render_desc* descs, uint32_t passes, kp_batch_tuning* out) {
     kp_ctx* c = b->c;
     const uint32_t tb_max = std::max(c->grid_closest5, c->grid_occluded5) / (uint32_t)c->cus;

@@ -669,16 +669,24 @@ static int guide_eval_common(kp_ctx* c, const float* in6, uint32_t n, float* out
     float* d_in3 = d_in + 6 * N;                       // directions or uniforms
     float* d_out = (float*)c->d_stage_out;             // outputs, densities or samples
     float* d_pdf = mode == 2 ? d_out + 3 * N : d_out;
-    KP_HIP_TRY(c, hipMemcpyAsync(d_in, in6, 6 * N * fl, hipMemcpyHostToDevice, c->stream));
-    if (mode != 0)
-        KP_HIP_TRY(c, hipMemcpyAsync(d_in3, mode == 1 ? dirs : u3, 3 * N * fl, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_guide_eval, dim3((n + 255) / 256), dim3(256), 0, c->stream, guide_net(c), d_in, n, d_out,
-                       d_in3, d_in3, d_out, d_pdf, mode);
-    KP_HIP_TRY(c, hipGetLastError());
-    if (mode == 0) KP_HIP_TRY(c, hipMemcpyAsync(out32, d_out, 32 * N * fl, hipMemcpyDeviceToHost, c->stream));
-    if (mode == 2) KP_HIP_TRY(c, hipMemcpyAsync(dirs_out, d_out, 3 * N * fl, hipMemcpyDeviceToHost, c->stream));
-    if (mode >= 1) KP_HIP_TRY(c, hipMemcpyAsync(pdf_out, d_pdf, N * fl, hipMemcpyDeviceToHost, c->stream));
-    KP_HIP_TRY(c, hipStreamSynchronize(c->stream));
+    hipError_t e = hipSuccess;
+    auto copy = [&](void* dst, const void* src, size_t floats, hipMemcpyKind kind) {
+        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, floats * fl, kind, c->stream);
+    };
+    copy(d_in, in6, 6 * N, hipMemcpyHostToDevice);
+    if (mode != 0) copy(d_in3, mode == 1 ? dirs : u3, 3 * N, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_guide_eval, dim3((n + 255) / 256), dim3(256), 0, c->stream, guide_net(c), d_in, n, d_out,
+                           d_in3, d_in3, d_out, d_pdf, mode);
+        e = hipGetLastError();
+    }
+    if (mode == 0) copy(out32, d_out, 32 * N, hipMemcpyDeviceToHost);
+    if (mode == 2) copy(dirs_out, d_out, 3 * N, hipMemcpyDeviceToHost);
+    if (mode >= 1) copy(pdf_out, d_pdf, N, hipMemcpyDeviceToHost);
+    // waited for after an error too: copies before it still use the caller's arrays
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return hip_fail(c, e, "guiding evaluation");
     return KP_OK;
 }
 
